@@ -52,6 +52,8 @@ __device__ __forceinline__ float dg_silu(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
 }
 
+#include "dense_few.h"
+
 template <int BM, int BN, int BK, int NW, int WR>
 struct Dg {
   static constexpr int NT = NW * 64;           // threads
@@ -719,10 +721,27 @@ __global__ __launch_bounds__(512, 1) void route_logits_kernel(const XT* __restri
 }
 
 // Logits [N][E] of any E (Epad = E rounded up to 16 rows of router_packed); xbf_out (fp32 x
-// only, may be null) receives x as bf16; zero[0 .. nzero) is cleared (null: nothing).
+// only, may be null) receives x as bf16, xfrag_out (may be null) x as bf16 in the small-batch
+// gate/up's operand order; zero[0 .. nzero) is cleared (null: nothing).
+// Up to RLF_MAX tokens take route_logits_few_kernel (the same bits): at H = 1536, E = 192 8.2
+// against 14.7 us at 16 tokens, the whole layer 91.2 -> 87.8 us at 509 (bf16 x), even at 1024
+// and 10 us slower at 2048, where every expert tile's workgroup reading its own x rows costs more
+// than the staging.
+#define RLF_MAX 512
 int pp_route_logits_dense(const void* x, int x_dtype, int64_t N, int H, const float* router, const float* bias,
-                          int E, float* logits_out, bf16_t* xbf_out, uint32_t* zero, int nzero, hipStream_t st) {
+                          int E, float* logits_out, bf16_t* xbf_out, uint32_t* zero, int nzero, hipStream_t st,
+                          bf16_t* xfrag_out) {
   if (N == 0) return PP_OK;
+  if (xfrag_out || N <= RLF_MAX) {
+    const dim3 grid((unsigned)((N + 15) / 16), (unsigned)((E + 15) / 16));
+    if (x_dtype == PP_DTYPE_F32)
+      route_logits_few_kernel<float><<<grid, 256, 0, st>>>((const float*)x, N, H, router, bias, E, logits_out, xbf_out,
+                                                           xfrag_out, zero, nzero);
+    else
+      route_logits_few_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)x, N, H, router, bias, E, logits_out,
+                                                            xbf_out, xfrag_out, zero, nzero);
+    return pp_check_launch("route_logits_few_kernel");
+  }
   const int Epad = (E + 15) / 16 * 16;
   const int te = E <= 16 ? 1 : E <= 32 ? 2 : 3;
   const dim3 grid((unsigned)((N + 16 * RL_TT - 1) / (16 * RL_TT)), (unsigned)((E + 16 * te - 1) / (16 * te)));
@@ -881,6 +900,45 @@ static int dense_gemm_launch(DgArgs a, hipStream_t st) {
   return pp_check_launch(MODE == 0 ? "dense_gemm_kernel (gate/up)" : "dense_gemm_kernel (down)");
 }
 
+// ------------------------------------------------------------------ small batches (dense_few.h)
+#define DF_R 2   // 16-row blocks per down workgroup
+#define DF_KW 3  // K steps per down wave
+static int few_parts(int I) { return (I / 32 + 8 * DF_KW - 1) / (8 * DF_KW); }
+
+struct FewWs {
+  int64_t h, part, total;  // floats from the start of the split workspace; xfrag at 0
+};
+static FewWs few_layout(int64_t n, int H, int I) {
+  const int64_t np = (n + 15) / 16 * 16;  // token rows padded to whole blocks
+  FewWs L;
+  L.h = np * H / 2;
+  L.part = L.h + np * I;
+  L.total = L.part + few_parts(I) * n * H;
+  return L;
+}
+
+// Layers of 17.4 MB (E = 192, G = 32, H = 1536; us, GEMM tiles -> this form): 83 -> 27 at 2
+// tokens, 82 -> 28.7 at 16, 84 -> 37.7 at 64, 84 -> 49 at 128, 88 -> 72 at 256, where each token
+// block still costs 2.9 us in all and the GEMM tiles' time has not begun to grow. H > 1536: the
+// weights no longer stay in registers over more than 64 tokens (H = 4096: 107 -> 84 at 64, 123 ->
+// 124 at 128). Buffers in the GEMMs' split workspace, which such a pass does not use.
+static bool dense_few_form(int64_t n, int H, int E, int G) {
+  return E != 16 && n <= (H <= 1536 ? DF_MAX : 64) &&
+         few_layout(n, H, E * G).total * 4 <= (int64_t)DG_MAX_GRID * (int64_t)DG_SLOT_BYTES;
+}
+
+static int dense_few_launch(const FewArgs& a, hipStream_t st) {
+  int rc;
+  const int units = a.I / 8;
+  if (a.H == 1536)  // six K steps a wave, all in registers
+    dense_few_gateup_kernel<3, 6, true><<<a.n_sel + (units + 2) / 3, 512, 0, st>>>(a);
+  else
+    dense_few_gateup_kernel<2, 6, false><<<a.n_sel + (units + 1) / 2, 512, 0, st>>>(a);
+  if ((rc = pp_check_launch("dense_few_gateup_kernel"))) return rc;
+  dense_few_down_kernel<DF_R, DF_KW><<<a.H / (16 * DF_R) * few_parts(a.I), 512, 0, st>>>(a);
+  return pp_check_launch("dense_few_down_kernel");
+}
+
 // One pass over n tokens (at most dense_pass_tokens). logits_out / mask_out (may be null)
 // receive the pass's routing.
 static int dense_pass(const void* x, int x_dtype, int64_t n, int H, const float* router, const float* bias, int E,
@@ -896,6 +954,9 @@ static int dense_pass(const void* x, int x_dtype, int64_t n, int H, const float*
   bf16_t* xbf_w = x_dtype == PP_DTYPE_BF16 ? nullptr : (bf16_t*)(ws + L.xbf);
   uint32_t* sync = (uint32_t*)(ws + L.sync);
   float* part = (float*)(ws + L.part);
+  const bool few = dense_few_form(n, H, E, G);
+  const bool sel_in = few && E > 64;  // the selection runs inside the gate/up launch
+  if (few) xbf_w = nullptr;
   if (E == 16) {  // the E = 16 router (the same logits as pp_route at E = 16)
     if ((rc = pp_route_impl(x, x_dtype, nullptr, n, H, router, bias, E, tau, logits, nullptr, gates, mask, nullptr,
                             xbf_w, st, nullptr)))
@@ -904,11 +965,34 @@ static int dense_pass(const void* x, int x_dtype, int64_t n, int H, const float*
     dg_zero_kernel<<<1, 256, 0, st>>>(sync, DG_SYNC_WORDS);
     if ((rc = pp_check_launch("dg_zero_kernel"))) return rc;
   } else {
-    if ((rc = pp_route_logits_dense(x, x_dtype, n, H, router, bias, E, logits, xbf_w, sync, DG_SYNC_WORDS, st)))
+    if ((rc = pp_route_logits_dense(x, x_dtype, n, H, router, bias, E, logits, xbf_w, sync, DG_SYNC_WORDS, st,
+                                    few ? (bf16_t*)part : nullptr)))
       return rc;
-    if ((rc = pp_route_impl(nullptr, PP_DTYPE_F32, logits, n, H, nullptr, nullptr, E, tau, nullptr, nullptr, gates,
-                            mask, nullptr, nullptr, st, nullptr)))
+    if (!sel_in && (rc = pp_route_impl(nullptr, PP_DTYPE_F32, logits, n, H, nullptr, nullptr, E, tau, nullptr, nullptr,
+                                       gates, mask, nullptr, nullptr, st, nullptr)))
       return rc;
+  }
+  if (few) {
+    FewArgs f;
+    const FewWs F = few_layout(n, H, E * G);
+    f.xfrag = (const bf16_t*)part;
+    f.rows = (const bf16_t*)packed;
+    f.down_t = (const bf16_t*)packed + (int64_t)E * G * 3 * H;
+    f.logits = logits;
+    f.gates = gates;
+    f.mask = mask;
+    f.h = part + F.h;
+    f.part = part + F.part;
+    f.tick = sync;
+    f.out = out;
+    f.tau = tau;
+    f.N = (int)n;
+    f.H = H;
+    f.E = E;
+    f.G = G;
+    f.I = E * G;
+    f.n_sel = sel_in ? (int)n : 0;
+    return dense_few_launch(f, st);
   }
   const int I = E * G, Ipad = pp_dense_ipad(E, G);
   bf16_t* act = (bf16_t*)(ws + L.act);

@@ -962,3 +962,41 @@ static __device__ void select_one_token_wg(LG lg, int E, float tau, SelScratch* 
     wg_lds_barrier();
   }
 }
+
+// One token's selection from its logits row by a workgroup of NT threads (route_select_wg_kernel
+// and the small-batch gate/up launch), outputs as pp_route's; null outputs are not written.
+struct SelWgScratch {
+  SelScratch ss;
+  unsigned long long keys[PP_MAX_EXPERTS];
+  float lg[PP_MAX_EXPERTS];
+  float red[8];
+};
+
+template <int NT>
+static __device__ __forceinline__ void route_select_wg_token(const float* __restrict__ logits, int64_t t, int E, float tau,
+                                             float* __restrict__ logits_copy, float* __restrict__ probs_out,
+                                             float* __restrict__ gates_out, uint8_t* __restrict__ mask_out,
+                                             int32_t* __restrict__ count_out, SelWgScratch* sc) {
+  static_assert(NT >= PP_MAX_EXPERTS && NT <= 512, "a thread per expert, a wave maximum per wave");
+  SelScratch& ss = sc->ss;
+  const int tid = threadIdx.x;
+  if (tid < E) {
+    sc->lg[tid] = logits[t * E + tid];
+    if (logits_copy) logits_copy[t * E + tid] = sc->lg[tid];
+  }
+  __syncthreads();
+  select_one_token_wg([&](int j) { return sc->lg[j]; }, E, tau, &ss, sc->keys, sc->red, tid, NT);
+  const bool bad = ss.bad != 0;
+  const int k = bad ? 0 : ss.k;
+  if (tid < E) ss.sel[tid] = 0;
+  __syncthreads();
+  if (tid < k) ss.sel[ss.order[tid]] = 1;
+  __syncthreads();
+  if (tid < E) {
+    const bool s = ss.sel[tid] != 0;
+    if (probs_out) probs_out[t * E + tid] = bad ? __builtin_nanf("") : ss.e[tid];
+    if (gates_out) gates_out[t * E + tid] = bad ? __builtin_nanf("") : (s ? pp_sigmoid(sc->lg[tid]) : 0.0f);
+    if (mask_out) mask_out[t * E + tid] = (uint8_t)s;
+  }
+  if (tid == 0 && count_out) count_out[t] = k;
+}

@@ -150,32 +150,9 @@ __global__ __launch_bounds__(256) void route_select_wg_kernel(const float* __res
                                                               float* __restrict__ gates_out,
                                                               uint8_t* __restrict__ mask_out,
                                                               int32_t* __restrict__ count_out) {
-  __shared__ SelScratch ss;
-  __shared__ unsigned long long keys_s[PP_MAX_EXPERTS];
-  __shared__ float lg_s[PP_MAX_EXPERTS];
-  __shared__ float red_s[4];
-  const int tid = threadIdx.x;
-  const int64_t t = blockIdx.x;
-  if (t >= N) return;  // uniform
-  if (tid < E) {
-    lg_s[tid] = logits[t * E + tid];
-    if (logits_copy) logits_copy[t * E + tid] = lg_s[tid];
-  }
-  __syncthreads();
-  select_one_token_wg([&](int j) { return lg_s[j]; }, E, tau, &ss, keys_s, red_s, tid, 256);
-  const bool bad = ss.bad != 0;
-  const int k = bad ? 0 : ss.k;
-  if (tid < E) ss.sel[tid] = 0;
-  __syncthreads();
-  if (tid < k) ss.sel[ss.order[tid]] = 1;
-  __syncthreads();
-  if (tid < E) {
-    const bool s = ss.sel[tid] != 0;
-    if (probs_out) probs_out[t * E + tid] = bad ? __builtin_nanf("") : ss.e[tid];
-    if (gates_out) gates_out[t * E + tid] = bad ? __builtin_nanf("") : (s ? pp_sigmoid(lg_s[tid]) : 0.0f);
-    if (mask_out) mask_out[t * E + tid] = (uint8_t)s;
-  }
-  if (tid == 0 && count_out) count_out[t] = k;
+  __shared__ SelWgScratch sc;
+  if ((int64_t)blockIdx.x >= N) return;  // uniform
+  route_select_wg_token<256>(logits, blockIdx.x, E, tau, logits_copy, probs_out, gates_out, mask_out, count_out, &sc);
 }
 
 // ------------------------------------------------------------------ E = 16 fast path
@@ -538,7 +515,8 @@ static void launch_route_few(const XT* x, int64_t N, int H, const float* router,
 // tokens, per expert, the number of selections -- the bucketing's block counts, so it
 // needs no counting pass.
 int pp_route_logits_dense(const void* x, int x_dtype, int64_t N, int H, const float* router, const float* bias,
-                          int E, float* logits_out, bf16_t* xbf_out, uint32_t* zero, int nzero, hipStream_t st);
+                          int E, float* logits_out, bf16_t* xbf_out, uint32_t* zero, int nzero, hipStream_t st,
+                          bf16_t* xfrag_out);
 
 int pp_route_impl(const void* x, int x_dtype, const float* logits_in, int64_t N, int H,
                   const float* router, const float* bias, int E, float tau, float* logits_out,
@@ -572,7 +550,7 @@ int pp_route_impl(const void* x, int x_dtype, const float* logits_in, int64_t N,
   if (!logits_in && logits_out) {
     // E != 16 with a logits buffer: the LDS-staged logits pass (one fixed summation order
     // per (token, expert), the prefill's own router), then the selection from those logits
-    int rc = pp_route_logits_dense(x, x_dtype, N, H, router, bias, E, logits_out, xbf_out, nullptr, 0, st);
+    int rc = pp_route_logits_dense(x, x_dtype, N, H, router, bias, E, logits_out, xbf_out, nullptr, 0, st, nullptr);
     if (rc) return rc;
     logits_in = logits_out;
     logits_out = nullptr;
