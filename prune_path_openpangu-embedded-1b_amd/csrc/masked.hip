@@ -14,15 +14,34 @@
 //   d_inter[n,d] = d_out[n,d] * gates[n, eid[d]]
 //   d_gates[n,e] = sum over the neurons d of expert e of d_out[n,d] * inter[n,d]
 // accumulated in fp32 in a fixed order, so repeated calls give the same bits: the
-// products are staged in LDS and summed through the expert-sorted neuron order (perm,
-// seg), TPE interleaved partial sums per expert then an xor tree, whatever the partition.
+// products are staged in LDS in the expert-sorted neuron order (perm, seg) and summed in
+// that order, TPE interleaved partial sums per expert then an xor tree, whatever the partition.
 //
 // Workgroups of 256 threads; each thread moves 8 consecutive elements per step (16-byte
 // bf16 / 32-byte fp32 vectors).
+#include <algorithm>
+
 #include "pp_common.h"
 
 #define MG_THREADS 256
-#define MG_MAX_I 16384  // LDS holds one row's fp32 products and the expert-sorted order (uint16)
+#define MG_MAX_I 16384  // LDS holds one row's fp32 products; places in the expert-sorted order are 16-bit
+
+// 16-byte loads and stores. Results are stored non-temporally: they are read next by another
+// kernel, after 100s of MB, and stored normally they take the place of the rows this launch still
+// has to read (16384 x 6144 bf16: forward 79.5 -> 57.3 us on rows that the cache could
+// hold). The backward is its rows' last reader and loads them non-temporally too (forward and
+// backward together 191 -> 175.7 us, 5.75 TB/s; the forward's loads left normal: 184.8 with them
+// non-temporal, as its backward reads them again).
+typedef uint32_t mg_u4 __attribute__((ext_vector_type(4)));
+template <bool NT>
+__device__ __forceinline__ uint4 mg_ld(const void* p) {
+  const mg_u4 v = NT ? __builtin_nontemporal_load((const mg_u4*)p) : *(const mg_u4*)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void mg_st(void* p, uint4 u) {
+  const mg_u4 v = {u.x, u.y, u.z, u.w};
+  __builtin_nontemporal_store(v, (mg_u4*)p);
+}
 
 template <typename T>
 struct MgVec;
@@ -33,8 +52,8 @@ struct MgVec<float> {
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
   }
   static __device__ __forceinline__ void store(float* p, const float (&v)[8]) {
-    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
-    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    mg_st(p, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
+    mg_st(p + 4, make_uint4(__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7])));
   }
   static __device__ __forceinline__ float gate(float g) { return g; }
 };
@@ -55,32 +74,34 @@ struct MgVec<bf16_t> {
     u.y = (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
     u.z = (uint32_t)f32_to_bf16(v[4]) | ((uint32_t)f32_to_bf16(v[5]) << 16);
     u.w = (uint32_t)f32_to_bf16(v[6]) | ((uint32_t)f32_to_bf16(v[7]) << 16);
-    *(uint4*)p = u;
+    mg_st(p, u);
   }
   static __device__ __forceinline__ float gate(float g) { return bf16_to_f32(f32_to_bf16(g)); }
 };
 
-// The backward is persistent over rows: a workgroup stages the neuron -> expert ids
-// (uint8) and the expert-sorted order (uint16) in LDS once and then takes rows
-// blockIdx.x, + gridDim.x, ...; the gates of the current row sit in one of two LDS
-// buffers (row parity). One workgroup per row re-read the order from L2 in a dependent
-// loop: 238 against 148 us for 16384 x 6144 bf16 at E = 16.
-__device__ __forceinline__ void mg_ids8(const uint8_t* e_s, int d, int (&e)[8]) {
-  const uint2 u = *(const uint2*)(e_s + d);
+// one row's elements of a thread in the storage type
+template <typename T, int NI>
+struct MgRow {
+  static constexpr int W = 8 * (int)sizeof(T) / 16;  // 16-byte words per 8 elements
+  uint4 v[NI][W];
+  template <bool NT>
+  __device__ __forceinline__ void load(const T* row, int tid, int I) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    e[i] = (u.x >> (8 * i)) & 0xff;
-    e[4 + i] = (u.y >> (8 * i)) & 0xff;
+    for (int it = 0; it < NI; ++it) {
+      const int d = 8 * tid + it * 8 * MG_THREADS;
+      if (d < I) {
+#pragma unroll
+        for (int q = 0; q < W; ++q) v[it][q] = mg_ld<NT>((const char*)(row + d) + 16 * q);
+      }
+    }
   }
-}
-
-__device__ __forceinline__ void mg_stage_ids(const int32_t* __restrict__ eid, int I, int E, uint8_t* e_s) {
-  for (int d = threadIdx.x; d < I; d += MG_THREADS)
-    e_s[d] = (uint8_t)min((unsigned)eid[d], (unsigned)(E - 1));  // ids come from the caller: clamped
-}
-
-#define MG_G_BYTES (2 * PP_MAX_EXPERTS * 4)
-static size_t mg_bwd_lds(int I) { return MG_G_BYTES + (size_t)I * 7 + (PP_MAX_EXPERTS + 1) * 4; }
+  __device__ __forceinline__ void get(int it, float (&f)[8]) const {
+    T t[8];
+#pragma unroll
+    for (int q = 0; q < W; ++q) *(uint4*)((char*)t + 16 * q) = v[it][q];
+    MgVec<T>::load(t, f);
+  }
+};
 
 // The forward takes one row per workgroup (no barrier between rows; the ids come
 // through L2 as int32 -- measured a little faster than the persistent form with the ids
@@ -105,7 +126,9 @@ __global__ __launch_bounds__(MG_THREADS) void masked_gate_fwd_kernel(const T* __
   for (int d = 8 * tid; d < I; d += 8 * MG_THREADS) {
     float v[8];
     int e[8];
-    MgVec<T>::load(inter + n * I + d, v);
+    MgRow<T, 1> xr;
+    xr.template load<false>(inter + n * I + d, 0, 8);
+    xr.get(0, v);
     mg_eids(eid, d, E, e);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = __fmul_rn(v[i], g_s[e[i]]);
@@ -113,60 +136,112 @@ __global__ __launch_bounds__(MG_THREADS) void masked_gate_fwd_kernel(const T* __
   }
 }
 
-// tpe: threads per expert for the sums (a power of two <= 64, E * tpe <= MG_THREADS).
-// LDS: gates [2][256], products fp32 [I], expert-sorted order uint16 [I], ids uint8 [I],
-// segments [E+1]. Per row: gates -> barrier -> d_inter and products -> barrier -> sums
-// (the next row's first barrier keeps its products from overwriting these).
+// ------------------------------------------------------------------ backward
+// Persistent over rows. A thread's elements are the same in every row (8 tid + 2048 it, NI
+// steps), so their expert ids and their places in the expert-sorted order are registers, and a
+// row is: products scattered to their sorted places in LDS, barrier, per-expert sums, barrier.
+// The next row's loads are issued before the first barrier and land under the sums (LDS-only
+// barriers: __syncthreads would wait for them).
+// Place k of the order sits at word MG_SKEW(k) = k + k / 32: the lanes of a wave sum segments 32 E' apart
+// (E = 192: 32 neurons each, one lane per expert), which would all start in two banks.
+// The earlier form kept the order and the ids in LDS (45 KB: three workgroups per CU), gathered
+// the products through the order (a dependent pair of LDS reads per term) and had no loads in
+// flight during the sums: 16384 x 6144 bf16, E = 16 / 192, 146 / 209 us, this form 126 / 132 with
+// the same loads and 111 / 117 with the non-temporal ones (5.4 / 5.2 TB/s); 6144 x 6144 fp32,
+// E = 192, 113 -> 93 us. Bound: memory (a copy of such rows reaches 5.1 to 6.2 TB/s).
+#define MG_SKEW(k) ((k) + ((k) >> 5))
+
+static size_t mg_bwd_lds(int I, int E) { return ((size_t)MG_SKEW(I) + 1 + 2 * E + E + 1) * 4; }
+
+// workgroups per CU (waves per SIMD) that the registers of NI steps leave room for
 template <typename T>
-__global__ __launch_bounds__(MG_THREADS) void masked_gate_bwd_kernel(
+constexpr int mg_bwd_wpc(int ni) {
+  return ni == 1 ? 6 : ni == 2 ? 5 : ni == 3 ? 4 : ni == 4 ? 3 : ni == 6 || sizeof(T) == 2 ? 2 : 1;
+}
+
+// tpe: threads per expert for the sums (a power of two <= 64, E * tpe <= MG_THREADS).
+template <typename T, int NI>
+__global__ __launch_bounds__(MG_THREADS, mg_bwd_wpc<T>(NI)) void masked_gate_bwd_kernel(
     const T* __restrict__ d_out, const T* __restrict__ inter, const float* __restrict__ gates,
     const int32_t* __restrict__ eid, const int32_t* __restrict__ perm, const int32_t* __restrict__ seg,
     int64_t n_rows, int I, int E, int tpe, T* __restrict__ d_inter, float* __restrict__ d_gates) {
-  extern __shared__ __align__(16) unsigned char mg_smem[];
-  float* g_s = (float*)mg_smem;
-  float* prod_s = (float*)(mg_smem + MG_G_BYTES);
-  uint16_t* p_s = (uint16_t*)(mg_smem + MG_G_BYTES + (size_t)I * 4);
-  uint8_t* e_s = mg_smem + MG_G_BYTES + (size_t)I * 6;
-  int* seg_s = (int*)(mg_smem + MG_G_BYTES + (size_t)I * 7);
+  extern __shared__ __align__(16) float mg_smem[];
+  const int np = MG_SKEW(I) + 1;  // sorted places, and one nobody sums
+  float* prod_s = mg_smem;
+  float* g_s = prod_s + np;        // [2][E]
+  int* seg_s = (int*)(g_s + 2 * E);
   const int tid = threadIdx.x;
-  mg_stage_ids(eid, I, E, e_s);
-  for (int k = tid; k < I; k += MG_THREADS) p_s[k] = (uint16_t)min((unsigned)perm[k], (unsigned)(I - 1));
-  for (int e = tid; e <= E; e += MG_THREADS) seg_s[e] = min(max(seg[e], 0), I);  // (clamped: from the caller)
-  const int ex = tid / tpe, j = tid - ex * tpe;
-  int par = 0;
-  for (int64_t n = blockIdx.x; n < n_rows; n += gridDim.x, par ^= 1) {
-    float* g = g_s + par * PP_MAX_EXPERTS;
-    for (int e = tid; e < E; e += MG_THREADS) g[e] = MgVec<T>::gate(gates[n * E + e]);
-    __syncthreads();
-    for (int d = 8 * tid; d < I; d += 8 * MG_THREADS) {
-      float go[8], x[8], gi[8];
-      int e[8];
-      MgVec<T>::load(d_out + n * I + d, go);
-      MgVec<T>::load(inter + n * I + d, x);
-      mg_ids8(e_s, d, e);
+  // the inverse of the order (ids, order and segments come from the caller: clamped)
+  uint16_t* inv_s = (uint16_t*)prod_s;
+  for (int k = tid; k < I; k += MG_THREADS) inv_s[k] = (uint16_t)(np - 1);
+  for (int e = tid; e <= E; e += MG_THREADS) seg_s[e] = min(max(seg[e], 0), I);
+  wg_lds_barrier();
+  for (int k = tid; k < I; k += MG_THREADS) inv_s[min((unsigned)perm[k], (unsigned)(I - 1))] = (uint16_t)MG_SKEW(k);
+  wg_lds_barrier();
+  uint32_t inv[NI][4];  // eight 16-bit places
+  uint32_t ids[NI][2];  // eight 8-bit expert ids
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        gi[i] = __fmul_rn(go[i], g[e[i]]);
-        prod_s[d + i] = __fmul_rn(go[i], x[i]);
-      }
-      if (d_inter) MgVec<T>::store(d_inter + n * I + d, gi);
+  for (int it = 0; it < NI; ++it) {
+    const int d = 8 * tid + it * 8 * MG_THREADS;
+    if (d < I) {
+      const uint4 p = *(const uint4*)(inv_s + d);
+      inv[it][0] = p.x, inv[it][1] = p.y, inv[it][2] = p.z, inv[it][3] = p.w;
+      int e[8];
+      mg_eids(eid, d, E, e);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        ids[it][h] = (uint32_t)e[4 * h] | (uint32_t)e[4 * h + 1] << 8 | (uint32_t)e[4 * h + 2] << 16 |
+                     (uint32_t)e[4 * h + 3] << 24;
     }
-    __syncthreads();
-    // expert ex, partial j over its neurons k = seg[ex] + j, + tpe, ... (expert-sorted
-    // order) in four interleaved sums, ((a0 + a1) + (a2 + a3)), then the xor tree
-    // inside the tpe-lane group
+  }
+  wg_lds_barrier();
+  for (int k = tid; k < np; k += MG_THREADS) prod_s[k] = 0.0f;
+  const int ex = tid / tpe, j = tid - ex * tpe;
+  MgRow<T, NI> go, x;
+  float gr = 0.0f;
+  auto load = [&](int64_t n) {
+    go.template load<true>(d_out + n * I, tid, I);
+    x.template load<true>(inter + n * I, tid, I);
+    if (tid < E) gr = gates[n * E + tid];
+  };
+  int64_t n = blockIdx.x;
+  if (n < n_rows) load(n);
+  for (int par = 0; n < n_rows; n += gridDim.x, par ^= 1) {
+    float* g = g_s + par * E;
+    if (tid < E) g[tid] = MgVec<T>::gate(gr);
+    wg_lds_barrier();  // gates visible; the previous row's sums done
+#pragma unroll
+    for (int it = 0; it < NI; ++it) {
+      const int d = 8 * tid + it * 8 * MG_THREADS;
+      if (d < I) {
+        float a[8], b[8], gi[8];
+        go.get(it, a);
+        x.get(it, b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          gi[i] = __fmul_rn(a[i], g[(ids[it][i >> 2] >> (8 * (i & 3))) & 0xff]);
+          prod_s[(inv[it][i >> 1] >> (16 * (i & 1))) & 0xffff] = __fmul_rn(a[i], b[i]);
+        }
+        if (d_inter) MgVec<T>::store(d_inter + n * I + d, gi);
+      }
+    }
+    if (n + gridDim.x < n_rows) load(n + gridDim.x);
+    wg_lds_barrier();
+    // expert ex, partial j over its places k = seg[ex] + j, + tpe, ... in four interleaved
+    // sums, ((a0 + a1) + (a2 + a3)), then the xor tree inside the tpe-lane group
     float s = 0.0f;
     if (ex < E) {
       const int k1 = seg_s[ex + 1];
       int k = seg_s[ex] + j;
       float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+#pragma unroll 2
       for (; k + 3 * tpe < k1; k += 4 * tpe) {
-        a0 = __fadd_rn(a0, prod_s[p_s[k]]);
-        a1 = __fadd_rn(a1, prod_s[p_s[k + tpe]]);
-        a2 = __fadd_rn(a2, prod_s[p_s[k + 2 * tpe]]);
-        a3 = __fadd_rn(a3, prod_s[p_s[k + 3 * tpe]]);
+        a0 = __fadd_rn(a0, prod_s[MG_SKEW(k)]);
+        a1 = __fadd_rn(a1, prod_s[MG_SKEW(k + tpe)]);
+        a2 = __fadd_rn(a2, prod_s[MG_SKEW(k + 2 * tpe)]);
+        a3 = __fadd_rn(a3, prod_s[MG_SKEW(k + 3 * tpe)]);
       }
-      for (; k < k1; k += tpe) a0 = __fadd_rn(a0, prod_s[p_s[k]]);
+      for (; k < k1; k += tpe) a0 = __fadd_rn(a0, prod_s[MG_SKEW(k)]);
       s = __fadd_rn(__fadd_rn(a0, a1), __fadd_rn(a2, a3));
     }
     for (int o = 1; o < tpe; o <<= 1) s = __fadd_rn(s, __shfl_xor(s, o, PP_WAVE));
@@ -174,13 +249,31 @@ __global__ __launch_bounds__(MG_THREADS) void masked_gate_bwd_kernel(
   }
 }
 
-// Workgroups per launch: as many as fit the CUs at the kernel's LDS use (at most 8 of
-// 256 threads per CU), no more than there are rows.
-static unsigned mg_grid(int64_t n_rows, size_t lds) {
-  int per_cu = (int)((160 * 1024) / (lds + 1024));
-  per_cu = per_cu < 1 ? 1 : per_cu > 8 ? 8 : per_cu;
-  const int64_t g = (int64_t)pp_device_cus() * per_cu;
-  return (unsigned)(n_rows < g ? n_rows : g);
+// Workgroups per launch: as many as fit the CUs by registers (wpc) and LDS, no more than
+// there are rows.
+static unsigned mg_grid(int64_t n_rows, size_t lds, int wpc) {
+  const int per_cu = std::max(1, std::min(wpc, (int)((160 * 1024) / (lds + 1024))));
+  return (unsigned)std::min<int64_t>(n_rows, (int64_t)pp_device_cus() * per_cu);
+}
+
+template <typename T>
+static void mg_bwd_launch(const void* d_out, const void* inter, const float* gates, const int32_t* eid,
+                          const int32_t* perm, const int32_t* seg, int64_t n_rows, int I, int E, void* d_inter,
+                          float* d_gates, hipStream_t st) {
+  int tpe = 64;
+  while (tpe > 1 && tpe * E > MG_THREADS) tpe >>= 1;
+  const size_t lds = mg_bwd_lds(I, E);
+  const int ni = (I + 8 * MG_THREADS - 1) / (8 * MG_THREADS);
+#define MG_BWD(NI)                                                                                                 \
+  masked_gate_bwd_kernel<T, NI><<<mg_grid(n_rows, lds, mg_bwd_wpc<T>(NI)), MG_THREADS, lds, st>>>(                 \
+      (const T*)d_out, (const T*)inter, gates, eid, perm, seg, n_rows, I, E, tpe, (T*)d_inter, d_gates)
+  if (ni <= 1) MG_BWD(1);
+  else if (ni <= 2) MG_BWD(2);
+  else if (ni <= 3) MG_BWD(3);
+  else if (ni <= 4) MG_BWD(4);
+  else if (ni <= 6) MG_BWD(6);
+  else MG_BWD(8);
+#undef MG_BWD
 }
 
 static int mg_check(const void* a, const void* b, int dtype, int64_t n_rows, int I, int E, const char* what) {
@@ -222,17 +315,9 @@ extern "C" int pp_masked_gate_bwd(const void* d_out, const void* inter, int dtyp
   PP_REQUIRE(((uintptr_t)d_inter & 15) == 0 && ((uintptr_t)expert_ids & 15) == 0, PP_ERR_INVALID,
              "pp_masked_gate_bwd: d_inter / expert_ids not 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  int tpe = 64;
-  while (tpe > 1 && tpe * E > MG_THREADS) tpe >>= 1;
-  const size_t lds = mg_bwd_lds(I);
-  const unsigned grid = mg_grid(n_rows, lds);
   if (dtype == PP_DTYPE_F32)
-    masked_gate_bwd_kernel<float><<<grid, MG_THREADS, lds, st>>>((const float*)d_out, (const float*)inter, gates,
-                                                                 expert_ids, perm, seg, n_rows, I, E, tpe,
-                                                                 (float*)d_inter, d_gates);
+    mg_bwd_launch<float>(d_out, inter, gates, expert_ids, perm, seg, n_rows, I, E, d_inter, d_gates, st);
   else
-    masked_gate_bwd_kernel<bf16_t><<<grid, MG_THREADS, lds, st>>>((const bf16_t*)d_out, (const bf16_t*)inter, gates,
-                                                                  expert_ids, perm, seg, n_rows, I, E, tpe,
-                                                                  (bf16_t*)d_inter, d_gates);
+    mg_bwd_launch<bf16_t>(d_out, inter, gates, expert_ids, perm, seg, n_rows, I, E, d_inter, d_gates, st);
   return pp_check_launch("pp_masked_gate_bwd");
 }
