@@ -24,6 +24,11 @@ __device__ __forceinline__ void gv_wait(u32x4& a0, u32x4& a1, u32x4& b0, u32x4& 
   asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a0), "+v"(a1), "+v"(b0), "+v"(b1) : "n"(N));
 }
 
+template <int N>
+__device__ __forceinline__ void gv_wait3(u32x4& a0, u32x4& b0, u32x4& b1) {
+  asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(a0), "+v"(b0), "+v"(b1) : "n"(N));
+}
+
 // 16-byte LDS read at a byte address, invisible to the compiler's memory model: it cannot
 // be ordered after (made to wait for) LDS-DMA writes the compiler sees as aliasing stores.
 // The caller orders it with its own waits (s_waitcnt vmcnt + s_barrier before, lds_wait_all

@@ -246,7 +246,7 @@ __global__ __launch_bounds__(GM_THREADS, 2) void down_kernel(
 // (wave tile 64 x 64), two workgroups per CU, persistent over (row tile, column tile)
 // items. Operands go straight from global memory into LDS (global_load_lds_dwordx4:
 // lane i of a wave writes bytes [16 i, 16 i + 16) of the wave's 1 KB block, no VGPR
-// staging) through GP_STAGES LDS stages; the DMA runs GP_STAGES - 1 K blocks ahead and
+// staging) through ST LDS stages; the DMA runs ST - 1 K blocks ahead and
 // does not stop at item boundaries -- the blocks of a workgroup's items form one
 // stream, so the next item's first blocks are in flight under the current item's last
 // MFMAs. Per-item data never stalls the stream: tile metadata comes through scalar
@@ -263,9 +263,9 @@ __global__ __launch_bounds__(GM_THREADS, 2) void down_kernel(
 // __syncthreads() adds a release fence that does the same. So fragment reads are
 // inline ds_read_b128 whose results are fenced by s_waitcnt lgkmcnt tied to the
 // fragment registers, and the per-K-block barrier waits only for this wave's DMA of
-// the block about to be read: every wave issues at least GP_DMA DMA instructions per
+// the block about to be read: every wave issues at least DMA (Gv) instructions per
 // block (past the last block it re-fetches that block into the free stage, never
-// read), so "at most GP_DMA * (GP_STAGES - 2) of this wave's vector memory ops
+// read), so "at most DMA * (ST - 2) of this wave's vector memory ops
 // outstanding" means its DMA of the block about to be read has landed (loads complete
 // in order; extra ops -- slot DMA, epilogue stores -- only make the wait stricter); the
 // barrier after it covers every wave and frees the stage written next.
@@ -298,18 +298,16 @@ __global__ __launch_bounds__(GM_THREADS, 2) void down_kernel(
 
 #define GP_BK 64         // K block (bf16 elements)
 #define GP_STAGES 2
+#define GP_NARROW_ST 3   // stages of the narrow gate/up tiles (24 KB each)
 #define GP_WG_PER_CU 2
 #define GP_ROWB (GP_BK * 2)                     // bytes of one tile row in a stage
 #define GP_CH (GP_BK / 8)                       // 16-byte chunks per row
 #define GP_TILE (128 * GP_ROWB)                 // one operand tile of one stage
-#define GP_STAGE (2 * GP_TILE)
 #define GP_RPI (1024 / GP_ROWB)                 // rows per DMA instruction (a wave's 1 KB)
 #define GP_NI (128 / (4 * GP_RPI))              // DMA instructions per tile per wave
-#define GP_DMA (2 * GP_NI)                      // per wave per K block (A + B)
 #define GP_KS (GP_BK / 16)                      // MFMA k-steps per K block
 #define GP_SLOT_BYTES 1024                      // per item: 128 token ids + 128 pair gates
 #define GP_NSLOT 4
-#define GP_LDS_BYTES (GP_STAGES * GP_STAGE + GP_NSLOT * GP_SLOT_BYTES)
 // chunk c of row r is stored at position c ^ gp_swz(r): any 16 consecutive rows of a
 // fragment read land in 16 distinct 16-byte slots of a 256-byte bank window
 __device__ __forceinline__ int gp_swz(int r) { return GP_BK == 64 ? (r >> 1) & 7 : (r >> 2) & 3; }
@@ -365,17 +363,29 @@ __device__ __forceinline__ bool gp_join(Get&& A, Set&& SET, const GpSched& sc, f
 
 // MODE 0: gate/up + SwiGLU (A = gathered x rows, B = gate/up rows of 64 neurons);
 // MODE 1: down (A = act rows, B = down_t rows of 128 hidden columns).
-template <int MODE>
-__global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
-    const bf16_t* __restrict__ abase, int H, int G, const bf16_t* __restrict__ bbase,
+// BN: B rows of a tile (2 x neurons, or hidden columns), 128 with the waves 2 x 2 or 64 with the
+// waves 4 x 1; ST: stages.
+template <int MODE, int BN, int ST>
+struct Gv {
+  static constexpr int WN = BN / 64;                    // wave columns
+  static constexpr int MI = WN;                         // 32-row blocks of a wave tile (128 WN / 4 rows)
+  static constexpr int NIB = BN / (4 * GP_RPI);         // B DMA instructions per wave per K block
+  static constexpr int DMA = GP_NI + NIB;
+  static constexpr int STAGE = GP_TILE + BN * GP_ROWB;
+  static constexpr int LDS = ST * STAGE + GP_NSLOT * GP_SLOT_BYTES;
+};
+
+template <int MODE, int BN, int ST>
+__device__ __forceinline__ void gemm_v3_body(
+    unsigned char* smem, const bf16_t* __restrict__ abase, int H, int G, const bf16_t* __restrict__ bbase,
     const int32_t* __restrict__ token_ids, const float* __restrict__ pair_gates,
     const int32_t* __restrict__ tiles, const int32_t* __restrict__ meta, bf16_t* __restrict__ act,
     float* __restrict__ y) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  unsigned char* slots = smem + GP_STAGES * GP_STAGE;
+  using V = Gv<MODE, BN, ST>;
+  unsigned char* slots = smem + ST * V::STAGE;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  const int n_ntile = MODE == 0 ? G / 64 : H / 128;
+  const int wm = w / V::WN, wn = w % V::WN;
+  const int n_ntile = MODE == 0 ? G / (BN / 2) : H / BN;
   const int K = MODE == 0 ? H : G;
   const int nkb = K / GP_BK;
   const int n_items = meta[0] * n_ntile;
@@ -402,7 +412,7 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
   };
 
   // issue cursor: row offsets of the item whose blocks are being issued
-  int64_t aoff[GP_NI], boff[GP_NI];
+  int64_t aoff[GP_NI], boff[V::NIB];
   auto setup_item = [&](int li) {
     const int item = sc.item(li);
     const int t = item / n_ntile, nt = item - t * n_ntile;
@@ -412,14 +422,18 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
     for (int i = 0; i < GP_NI; ++i) {
       const int r = (4 * i + w) * GP_RPI + lane / GP_CH;
       const int pchunk = ((lane % GP_CH) ^ gp_swz(r)) * 8;
+      aoff[i] = MODE == 0 ? (int64_t)tok[r] * H + pchunk : (int64_t)(p0 + min(r, rows - 1)) * G + pchunk;
+    }
+#pragma unroll
+    for (int i = 0; i < V::NIB; ++i) {
+      const int r = (4 * i + w) * GP_RPI + lane / GP_CH;
+      const int pchunk = ((lane % GP_CH) ^ gp_swz(r)) * 8;
       if (MODE == 0) {
-        aoff[i] = (int64_t)tok[r] * H + pchunk;
-        // B tile row r = wn_*64 + j*32 + q -> gate (j=0) / up (j=1) row of neuron nt*64 + wn_*32 + q
+        // B tile row r = wn_*64 + j*32 + q -> gate (j=0) / up (j=1) row of neuron nt*BN/2 + wn_*32 + q
         const int wn_ = r >> 6, j = (r >> 5) & 1, q = r & 31;
-        boff[i] = ((int64_t)(e * G + nt * 64 + wn_ * 32 + q) * 3 + j) * H + pchunk;
+        boff[i] = ((int64_t)(e * G + nt * (BN / 2) + wn_ * 32 + q) * 3 + j) * H + pchunk;
       } else {
-        aoff[i] = (int64_t)(p0 + min(r, rows - 1)) * G + pchunk;
-        boff[i] = ((int64_t)e * H + nt * 128 + r) * G + pchunk;
+        boff[i] = ((int64_t)e * H + nt * BN + r) * G + pchunk;
       }
     }
   };
@@ -432,12 +446,12 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
       // prologue (the first item's blocks may all be in flight before its first wait)
       if (li >= 1 && li + 1 < n_local_items) slot_dma(li + 1);
     }
-    unsigned char* sb = smem + (f % GP_STAGES) * GP_STAGE;
+    unsigned char* sb = smem + (f % ST) * V::STAGE;
 #pragma unroll
     for (int i = 0; i < GP_NI; ++i) {
       const int blk = (4 * i + w) * 1024;
       gl2lds(abase + aoff[i] + kb * GP_BK, sb + blk);
-      gl2lds(bbase + boff[i] + kb * GP_BK, sb + GP_TILE + blk);
+      if (i < V::NIB) gl2lds(bbase + boff[i < V::NIB ? i : 0] + kb * GP_BK, sb + GP_TILE + blk);
     }
   };
 
@@ -447,7 +461,7 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
   for (int ks = 0; ks < GP_KS; ++ks) {
     const int r = lane & 31, c = ks * 2 + (lane >> 5);
     const uint32_t o = (uint32_t)(r * GP_CH + (c ^ gp_swz(r))) * 16;
-    offA[ks] = lds0 + wm * 64 * GP_ROWB + o;
+    offA[ks] = lds0 + wm * (32 * V::MI) * GP_ROWB + o;
     offB[ks] = lds0 + GP_TILE + wn * 64 * GP_ROWB + o;
   }
 
@@ -456,39 +470,41 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
   if (n_local_items > 1) slot_dma(1);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-  for (int f = 0; f < GP_STAGES - 1; ++f) issue(f);
+  for (int f = 0; f < ST - 1; ++f) issue(f);
 
-  f32x16_t acc[2][2];
+  f32x16_t acc[V::MI][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < V::MI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
 
   for (int f = 0; f < F; ++f) {
-    gp_wait_barrier<GP_DMA * (GP_STAGES - 2)>();
-    issue(f + GP_STAGES - 1);
-    const uint32_t sbase = (f % GP_STAGES) * GP_STAGE;
-    u32x4 fa[2][2], fb[2][2];
-    fa[0][0] = gv_read<0>(offA[0] + sbase);
-    fa[0][1] = gv_read<32 * GP_ROWB>(offA[0] + sbase);
-    fb[0][0] = gv_read<0>(offB[0] + sbase);
-    fb[0][1] = gv_read<32 * GP_ROWB>(offB[0] + sbase);
+    gp_wait_barrier<V::DMA * (ST - 2)>();
+    issue(f + ST - 1);
+    const uint32_t sbase = (f % ST) * V::STAGE;
+    u32x4 fa[2][V::MI], fb[2][2];
+    auto rd = [&](int ks, u32x4(&a)[V::MI], u32x4(&b)[2]) {
+      a[0] = gv_read<0>(offA[ks] + sbase);
+      if constexpr (V::MI == 2) a[1] = gv_read<32 * GP_ROWB>(offA[ks] + sbase);
+      b[0] = gv_read<0>(offB[ks] + sbase);
+      b[1] = gv_read<32 * GP_ROWB>(offB[ks] + sbase);
+    };
+    rd(0, fa[0], fb[0]);
 #pragma unroll
     for (int ks = 0; ks < GP_KS; ++ks) {
       const int cur = ks & 1, nxt = cur ^ 1;
-      if (ks < GP_KS - 1) {
-        fa[nxt][0] = gv_read<0>(offA[ks + 1] + sbase);
-        fa[nxt][1] = gv_read<32 * GP_ROWB>(offA[ks + 1] + sbase);
-        fb[nxt][0] = gv_read<0>(offB[ks + 1] + sbase);
-        fb[nxt][1] = gv_read<32 * GP_ROWB>(offB[ks + 1] + sbase);
-        gv_wait<4>(fa[cur][0], fa[cur][1], fb[cur][0], fb[cur][1]);
+      if (ks < GP_KS - 1) rd(ks + 1, fa[nxt], fb[nxt]);
+      if constexpr (V::MI == 2) {
+        if (ks < GP_KS - 1) gv_wait<4>(fa[cur][0], fa[cur][1], fb[cur][0], fb[cur][1]);
+        else gv_wait<0>(fa[cur][0], fa[cur][1], fb[cur][0], fb[cur][1]);
       } else {
-        gv_wait<0>(fa[cur][0], fa[cur][1], fb[cur][0], fb[cur][1]);
+        if (ks < GP_KS - 1) gv_wait3<3>(fa[cur][0], fb[cur][0], fb[cur][1]);
+        else gv_wait3<0>(fa[cur][0], fb[cur][0], fb[cur][1]);
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < V::MI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = mfma32v(fa[cur][i], fb[cur][j], acc[i][j]);
     }
@@ -505,31 +521,31 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
       const int p0 = tiles[t * 4 + 1], rows = tiles[t * 4 + 2];
       if (MODE == 0) {
         const float* gts = (const float*)(slots + (li & (GP_NSLOT - 1)) * GP_SLOT_BYTES + 512);
-        const int neuron = nt * 64 + wn * 32 + (ln & 31);
+        const int neuron = nt * (BN / 2) + wn * 32 + (ln & 31);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < V::MI; ++i)
 #pragma unroll
           for (int q = 0; q < 16; ++q) {
-            const int r = wm * 64 + i * 32 + mfma32_row(q, ln);
+            const int r = wm * (32 * V::MI) + i * 32 + mfma32_row(q, ln);
             if (r < rows)
               act[(int64_t)(p0 + r) * G + neuron] = f32_to_bf16(pp_silu(acc[i][0][q]) * acc[i][1][q] * gts[r]);
           }
       } else {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < V::MI; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
-            const int h = nt * 128 + wn * 64 + j * 32 + (ln & 31);
+            const int h = nt * BN + wn * 64 + j * 32 + (ln & 31);
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-              const int r = wm * 64 + i * 32 + mfma32_row(q, ln);
+              const int r = wm * (32 * V::MI) + i * 32 + mfma32_row(q, ln);
               if (r < rows) y[(int64_t)(p0 + r) * H + h] = acc[i][j][q];
             }
           }
       }
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < V::MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -537,6 +553,26 @@ __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
   }
   // the redundant tail DMAs must land before the workgroup's LDS is released
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// gate/up with at most narrow_max (one per CU) 64-neuron items takes 32-neuron tiles: twice the
+// items, and three stages where the wide tile has two. With a workgroup alone on its CU a K block
+// is a DMA latency, not bandwidth or MFMA work: at E = 16, G = 384, H = 1536 the gate/up launch
+// takes 27 -> 17.5 us at 128 tokens (96 wide items; two stages 24, four or six 17), 28 -> 25.4 at 333
+// (144: some CUs then hold two narrow items), the layer 56.1 -> 45.4 and 54.0 -> 50.5; from 192
+// wide items (500 tokens) on both take the same, past one per CU the narrow tile's second
+// reading of A costs (800 tokens 72.7 -> 75.4).
+template <int MODE>
+__global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
+    const bf16_t* __restrict__ abase, int H, int G, const bf16_t* __restrict__ bbase,
+    const int32_t* __restrict__ token_ids, const float* __restrict__ pair_gates,
+    const int32_t* __restrict__ tiles, const int32_t* __restrict__ meta, bf16_t* __restrict__ act,
+    float* __restrict__ y, int narrow_max) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (MODE == 0 && meta[0] * (G / 64) <= narrow_max)
+    gemm_v3_body<0, 64, GP_NARROW_ST>(smem, abase, H, G, bbase, token_ids, pair_gates, tiles, meta, act, y);
+  else
+    gemm_v3_body<MODE, 128, GP_STAGES>(smem, abase, H, G, bbase, token_ids, pair_gates, tiles, meta, act, y);
 }
 
 // ------------------------------------------------------------------ short tiles
@@ -816,9 +852,10 @@ static int gateup_launch(const bf16_t* xb, int H, int G, const bf16_t* wrows, in
     gemm_s_kernel<0><<<gemm_s_grid(), GM_THREADS, GS_LDS_BYTES, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles,
                                                                       meta, act, nullptr, part, sync);
   } else if (G % 64 == 0) {
-    int grid = gemm_grid_v3(max_tiles * (G / 64));
-    gemm_v3_kernel<0><<<grid, GM_THREADS, GP_LDS_BYTES, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles, meta,
-                                                              act, nullptr);
+    int grid = gemm_grid_v3(max_tiles * (G / 32));
+    constexpr int lds = std::max(Gv<0, 128, GP_STAGES>::LDS, Gv<0, 64, GP_NARROW_ST>::LDS);
+    gemm_v3_kernel<0><<<grid, GM_THREADS, lds, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles, meta, act, nullptr,
+                                                     pp_device_cus());
   } else {
     int grid = gemm_grid(max_tiles * (G / 32));
     gateup_kernel<4, 1, 1><<<grid, GM_THREADS, 0, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles, meta, act);
@@ -837,8 +874,8 @@ static int down_launch(const bf16_t* act, int H, int G, const bf16_t* down_t, co
                                                                       meta, nullptr, y, part, sync);
   } else if (G % 64 == 0) {
     int grid = gemm_grid_v3(max_tiles * (H / 128));
-    gemm_v3_kernel<1><<<grid, GM_THREADS, GP_LDS_BYTES, st>>>(act, H, G, down_t, nullptr, nullptr, tiles, meta,
-                                                              nullptr, y);
+    gemm_v3_kernel<1><<<grid, GM_THREADS, Gv<1, 128, GP_STAGES>::LDS, st>>>(act, H, G, down_t, nullptr, nullptr, tiles,
+                                                                            meta, nullptr, y, 0);
   } else {
     int grid = gemm_grid(max_tiles * (H / 128));
     down_kernel<<<grid, GM_THREADS, 0, st>>>(act, H, G, down_t, tiles, meta, y);
