@@ -247,16 +247,20 @@ int pp_moe_decode_batch(const void* x, int x_dtype, int64_t n_tokens, int H, con
  *     (bf16 MFMA) -> grouped down GEMM -> per-token combine in fp32 -> bf16. The pair
  *     buffers are sized for every token selecting every expert, so the call runs in
  *     consecutive passes of at most max(64, 512 MiB / (E * H * 4)) tokens (2048 tokens in
- *     one pass at E = 16, H = 1536).
+ *     one pass at E = 16, H = 1536). At E = 16, calls longer than that (and from 2048 tokens
+ *     on with tau >= 0.9) may instead take one down GEMM over every expert, the acts of the
+ *     experts a token does not select being 0: chosen on the device, per pass, from the
+ *     number of selected pairs; passes of up to 8192 tokens on the same workspace.
  *   G % 64 != 0 (e.g. the checkpoint's E = 192 experts of G = 32 neurons, narrower than an
  *     MFMA column tile): router logits (fp32 MFMA, one fixed summation order per
  *     (token, expert): a token routes the same way in any batch) -> selection -> dense
  *     gate/up GEMM over every (token, neuron) with act = bf16(silu(g) * u * gate), 0 for the
  *     experts a token does not select -> dense down GEMM over all neurons, fp32
- *     accumulation, one rounding to bf16. Passes of up to ~256 MiB of per-token buffers
- *     (about 15000 tokens at H = 1536, E = 192, G = 32).
- * Either way the output is the same as one pass over all N, and the same bits on every
- * call with the same N.
+ *     accumulation, one rounding to bf16. Up to 256 tokens (64 above H = 1536): the same
+ *     arithmetic in three launches that stream the weights. Passes of up to ~256 MiB of
+ *     per-token buffers (about 15000 tokens at H = 1536, E = 192, G = 32).
+ * Either way every token's routing is the same as in one pass over all N (its sums may be
+ * taken in another order), and the output is the same bits on every call with the same N.
  * workspace: pp_prefill_workspace_bytes(N, H, E, G) bytes of device scratch.
  * ------------------------------------------------------------------------- */
 size_t pp_prefill_workspace_bytes(int64_t n_tokens, int H, int E, int G);

@@ -88,6 +88,13 @@ struct DgArgs {
   int64_t N;
   int H, E, G, I, Ipad;
   int ct_lo, ct_hi;  // column tiles [ct_lo, ct_hi) of the launch's tile width
+  // ALL: with fewer than min_pairs pairs
+  // (bucketing's meta) the launch is the grouped pipeline's combine of y instead
+  const int32_t* meta;
+  int min_pairs;
+  const uint8_t* mask;  // [N][E]
+  const float* y;
+  const int32_t *token_pairs, *count;
 };
 
 // Wait until at most N LDS reads are outstanding, then tie the fragments of the current
@@ -140,7 +147,9 @@ __device__ __forceinline__ void dg_tile(int item, int n_rt, int n_ct, int gr, in
   rt = q * gr + (r - ctl * rows);
 }
 
-template <int MODE, int BM, int BN, int BK, int STAGES, int NW, int WR, int WPC>
+// ALL (MODE 1): the E = 16 prefill's launch, with the other uses of DgArgs::meta; a template
+// parameter, as the code alone cost the dense form's down launch 1 us.
+template <int MODE, int BM, int BN, int BK, int STAGES, int NW, int WR, int WPC, bool ALL>
 __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
   using C = Dg<BM, BN, BK, NW, WR>;
   constexpr int NB2 = BN / 2;  // MODE 0: neurons of a column tile (their gate and up rows)
@@ -158,6 +167,10 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int role_s;
   __shared__ float gate_s[MODE == 0 ? BM * GX : 1];  // MODE 0 epilogue: the tile's router gates
+  if (ALL && p.meta[1] < p.min_pairs) {  // uniform
+    combine_rows<NW * 64, 2>(p.y, p.token_pairs, p.count, p.N, p.H, p.E, p.out);
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in an SGPR
   const int wm = w / C::WN, wn = w % C::WN;
@@ -168,6 +181,7 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
   const GpSched sc(n_items, nkb, p.sync != nullptr, DG_NPMAX);
   const int F = sc.units(nkb);
   if (F <= 0) return;
+  bool odd = false;  // ALL: a result of this thread is infinite or NaN
 
   // ---- DMA issue cursor. Wave w, instruction i covers tile rows (NW i + w) * RPI .. + RPI;
   // lane l takes row (NW i + w) * RPI + l / CH and LDS chunk position l % CH, i.e. global
@@ -443,6 +457,7 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
               } else {
                 const int hc = ct * BN + wn * C::WC + col;
                 if (hc < p.H) p.out[(t0 + rl) * p.H + hc] = f32_to_bf16(sv[h]);
+                if (ALL) odd |= !(__builtin_fabsf(sv[h]) < __builtin_huge_valf());
               }
             }
           }
@@ -510,6 +525,7 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
                 for (int q = 0; q < 16; ++q) {
                   const int rl = i * 32 + mfma32_row(q, ln);
                   *(bf16_t*)(ep + (rl - hf * RP) * RW + (nl - jg * 32) * 2) = f32_to_bf16(v[q]);
+                  if (ALL) odd |= !(__builtin_fabsf(v[q]) < __builtin_huge_valf());
                 }
               }
             }
@@ -530,6 +546,31 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
   }
   // the redundant tail DMAs must land before the workgroup's LDS is released
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (ALL && __syncthreads_or(odd)) {
+    // Infinite or NaN results again, over the selected experts alone: the others' acts are 0, and 0
+    // times an infinite or NaN weight is NaN. Every element of the workgroup's tiles is looked at
+    // (of a split tile also those that other workgroups reduce: they do the same after their own
+    // stores, and write the same values).
+    for (int li = 0; li < n_local; ++li) {
+      int ctl, rt;
+      dg_tile(sc.item(li), n_rt, n_ct, DG_DN_GR, rt, ctl);
+      for (int i = tid; i < BM * BN; i += C::NT) {
+        const int64_t t = (int64_t)rt * BM + i / BN;
+        const int h = (p.ct_lo + ctl) * BN + i % BN;
+        if (t >= p.N || h >= p.H || (p.out[t * p.H + h] & 0x7f80u) != 0x7f80u) continue;
+        float s = 0.0f;
+        for (int e = 0; e < p.E; ++e) {
+          if (!p.mask[t * p.E + e]) continue;
+          const bf16_t* av = p.a + t * p.Ipad + e * p.G;
+          const bf16_t* wv = p.b + ((int64_t)e * p.H + h) * p.G;
+          float d = 0.0f;
+          for (int g = 0; g < p.G; ++g) d = fmaf(bf16_to_f32(av[g]), bf16_to_f32(wv[g]), d);
+          s += d;
+        }
+        p.out[t * p.H + h] = f32_to_bf16(s);
+      }
+    }
+  }
 }
 
 // ------------------------------------------------------------------ router logits (E > 16)
@@ -892,10 +933,10 @@ static int dense_grid() {
   return std::max(8, std::min(DG_MAX_GRID, g));
 }
 
-template <int MODE, int BM, int BN, int BK, int ST, int NW, int WR, int WPC>
+template <int MODE, int BM, int BN, int BK, int ST, int NW, int WR, int WPC, bool ALL = false>
 static int dense_gemm_launch(DgArgs a, hipStream_t st) {
   if (WPC > 1) a.part = nullptr, a.sync = nullptr;  // the split slots are sized for dense_grid() parts
-  dense_gemm_kernel<MODE, BM, BN, BK, ST, NW, WR, WPC>
+  dense_gemm_kernel<MODE, BM, BN, BK, ST, NW, WR, WPC, ALL>
       <<<dense_grid() * WPC, NW * 64, ST * Dg<BM, BN, BK, NW, WR>::STAGE, st>>>(a);
   return pp_check_launch(MODE == 0 ? "dense_gemm_kernel (gate/up)" : "dense_gemm_kernel (down)");
 }
@@ -1036,6 +1077,36 @@ static int dense_pass(const void* x, int x_dtype, int64_t n, int H, const float*
   a.ct_lo = 0;
   a.ct_hi = (H + DG_DN_BN - 1) / DG_DN_BN;
   return dense_gemm_launch<1, DG_DN_BM, DG_DN_BN, DG_DN_BK, DG_DN_ST, DG_DN_NW, DG_DN_WR, DG_DN_WPC>(a, st);
+}
+
+// The down projection of the grouped prefill over every expert at once (see prefill.hip), or its
+// combine: act [n][I], 0 for the experts a token does not select, out bf16 [n][H]. sync:
+// pp_dense_split_words words, zero at launch; part: pp_dense_split_bytes.
+size_t pp_dense_split_bytes() { return (size_t)DG_MAX_GRID * DG_SLOT_BYTES; }
+int pp_dense_split_words() { return DG_SYNC_WORDS / 2; }
+int pp_dense_down(const bf16_t* act, int64_t n, int H, int E, int G, const bf16_t* down_t, bf16_t* out,
+                  uint32_t* sync, float* part, const int32_t* meta, int min_pairs, const uint8_t* mask,
+                  const float* y, const int32_t* token_pairs, const int32_t* count, hipStream_t st) {
+  DgArgs a = {};
+  a.a = act;
+  a.b = down_t;
+  a.out = out;
+  a.part = part;
+  a.sync = sync;
+  a.N = n;
+  a.H = H;
+  a.E = E;
+  a.G = G;
+  a.I = E * G;
+  a.Ipad = pp_dense_ipad(E, G);
+  a.ct_hi = (H + DG_DN_BN - 1) / DG_DN_BN;
+  a.meta = meta;
+  a.min_pairs = min_pairs;
+  a.mask = mask;
+  a.y = y;
+  a.token_pairs = token_pairs;
+  a.count = count;
+  return dense_gemm_launch<1, DG_DN_BM, DG_DN_BN, DG_DN_BK, DG_DN_ST, DG_DN_NW, DG_DN_WR, DG_DN_WPC, true>(a, st);
 }
 
 // The whole dense-form prefill over N tokens in passes (inputs validated by the caller).

@@ -142,3 +142,71 @@ struct GpSched {
   }
 };
 
+// ------------------------------------------------------------------ combine
+// Per (token, 8 columns): the token's pair ids are read first (one batch of independent
+// loads), then up to CB_BATCH y rows at once, summed in expert order: two memory round
+// trips per batch instead of two per pair.
+#define CB_BATCH 8
+// U such columns per thread at once (NT threads a workgroup).
+template <int NT, int U>
+__device__ __forceinline__ void combine_rows(const float* __restrict__ y, const int32_t* __restrict__ token_pairs,
+                                             const int32_t* __restrict__ count, int64_t N, int H, int E,
+                                             bf16_t* __restrict__ out) {
+  const int HC = H >> 3;
+  const int64_t total = N * HC, step = (int64_t)gridDim.x * NT;
+  for (int64_t i0 = (int64_t)blockIdx.x * NT + threadIdx.x; i0 < total; i0 += U * step) {
+    int64_t t[U];
+    int ch[U], k[U], kmax = 0;
+    float4 s0[U], s1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = min(i0 + u * step, total - 1);  // past the end: the last one again, not stored
+      t[u] = i / HC;
+      ch[u] = (int)(i % HC);
+      s0[u] = s1[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      k[u] = min(count[t[u]], E);
+      kmax = max(kmax, k[u]);
+    }
+    for (int q0 = 0; q0 < kmax; q0 += CB_BATCH) {
+      int p[U][CB_BATCH];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < CB_BATCH; ++j) p[u][j] = q0 + j < k[u] ? token_pairs[t[u] * E + q0 + j] : -1;
+      float4 a[U][CB_BATCH], b[U][CB_BATCH];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < CB_BATCH; ++j)
+          // a negative id (fewer pairs than count: inconsistent caller data) ends the sum;
+          // nothing is read out of range
+          if (p[u][j] >= 0) {
+            const float4* src = (const float4*)(y + (int64_t)p[u][j] * H + ch[u] * 8);
+            a[u][j] = src[0];
+            b[u][j] = src[1];
+          }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < CB_BATCH; ++j) {
+          if (q0 + j >= k[u]) break;
+          if (p[u][j] < 0) {
+            k[u] = 0;
+            break;
+          }
+          s0[u].x += a[u][j].x; s0[u].y += a[u][j].y; s0[u].z += a[u][j].z; s0[u].w += a[u][j].w;
+          s1[u].x += b[u][j].x; s1[u].y += b[u][j].y; s1[u].z += b[u][j].z; s1[u].w += b[u][j].w;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i0 + u * step >= total) break;
+      uint4 o;
+      o.x = (uint32_t)f32_to_bf16(s0[u].x) | ((uint32_t)f32_to_bf16(s0[u].y) << 16);
+      o.y = (uint32_t)f32_to_bf16(s0[u].z) | ((uint32_t)f32_to_bf16(s0[u].w) << 16);
+      o.z = (uint32_t)f32_to_bf16(s1[u].x) | ((uint32_t)f32_to_bf16(s1[u].y) << 16);
+      o.w = (uint32_t)f32_to_bf16(s1[u].z) | ((uint32_t)f32_to_bf16(s1[u].w) << 16);
+      *(uint4*)(out + t[u] * H + ch[u] * 8) = o;
+    }
+  }
+}

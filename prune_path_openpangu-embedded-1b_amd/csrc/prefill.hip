@@ -16,6 +16,8 @@
 // beyond the last partial tile of each expert), 256 threads = 4 waves, BK = 64:
 // gemm_v3_kernel for G % 64 == 0 (LDS-DMA pipeline, below), gateup_kernel /
 // down_kernel (register-staged, row-padded LDS tiles) otherwise.
+#include <limits.h>
+
 #include <algorithm>
 
 #include "pp_common.h"
@@ -375,12 +377,12 @@ struct Gv {
   static constexpr int LDS = ST * STAGE + GP_NSLOT * GP_SLOT_BYTES;
 };
 
-template <int MODE, int BN, int ST>
+template <int MODE, int BN, int ST, bool ALL>
 __device__ __forceinline__ void gemm_v3_body(
     unsigned char* smem, const bf16_t* __restrict__ abase, int H, int G, const bf16_t* __restrict__ bbase,
     const int32_t* __restrict__ token_ids, const float* __restrict__ pair_gates,
     const int32_t* __restrict__ tiles, const int32_t* __restrict__ meta, bf16_t* __restrict__ act,
-    float* __restrict__ y) {
+    float* __restrict__ y, int act_ld) {
   using V = Gv<MODE, BN, ST>;
   unsigned char* slots = smem + ST * V::STAGE;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -519,7 +521,19 @@ __device__ __forceinline__ void gemm_v3_body(
       asm volatile("" : "+v"(ln));
       const int t = item / n_ntile, nt = item - t * n_ntile;
       const int p0 = tiles[t * 4 + 1], rows = tiles[t * 4 + 2];
-      if (MODE == 0) {
+      if (ALL && MODE == 0 && act_ld) {  // act rows by token: its expert's columns of [N][act_ld]
+        const int32_t* tok = (const int32_t*)(slots + (li & (GP_NSLOT - 1)) * GP_SLOT_BYTES);
+        const float* gts = (const float*)tok + 128;
+        bf16_t* col = act + tiles[t * 4 + 0] * G + nt * (BN / 2) + wn * 32 + (ln & 31);
+#pragma unroll
+        for (int i = 0; i < V::MI; ++i)
+#pragma unroll
+          for (int q = 0; q < 16; ++q) {
+            const int r = wm * (32 * V::MI) + i * 32 + mfma32_row(q, ln);
+            if (r < rows)
+              col[(int64_t)tok[r] * act_ld] = f32_to_bf16(pp_silu(acc[i][0][q]) * acc[i][1][q] * gts[r]);
+          }
+      } else if (MODE == 0) {
         const float* gts = (const float*)(slots + (li & (GP_NSLOT - 1)) * GP_SLOT_BYTES + 512);
         const int neuron = nt * (BN / 2) + wn * 32 + (ln & 31);
 #pragma unroll
@@ -562,17 +576,22 @@ __device__ __forceinline__ void gemm_v3_body(
 // (144: some CUs then hold two narrow items), the layer 56.1 -> 45.4 and 54.0 -> 50.5; from 192
 // wide items (500 tokens) on both take the same, past one per CU the narrow tile's second
 // reading of A costs (800 tokens 72.7 -> 75.4).
-template <int MODE>
+// NARROW and ALL (the down projection over every expert may follow) are template parameters, so
+// that the calls that need neither run the smaller code (0.5 % of the layer at 2048 tokens).
+template <int MODE, bool NARROW, bool ALL>
 __global__ __launch_bounds__(GM_THREADS, GP_WG_PER_CU) void gemm_v3_kernel(
     const bf16_t* __restrict__ abase, int H, int G, const bf16_t* __restrict__ bbase,
     const int32_t* __restrict__ token_ids, const float* __restrict__ pair_gates,
     const int32_t* __restrict__ tiles, const int32_t* __restrict__ meta, bf16_t* __restrict__ act,
-    float* __restrict__ y, int narrow_max) {
+    float* __restrict__ y, int narrow_max, int min_pairs, int I) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (MODE == 0 && meta[0] * (G / 64) <= narrow_max)
-    gemm_v3_body<0, 64, GP_NARROW_ST>(smem, abase, H, G, bbase, token_ids, pair_gates, tiles, meta, act, y);
+  const bool by_token = ALL && meta[1] >= min_pairs;  // the down projection over every expert follows
+  if (MODE == 1 && by_token) return;
+  const int act_ld = by_token ? I : 0;
+  if (NARROW && meta[0] * (G / 64) <= narrow_max)
+    gemm_v3_body<0, 64, GP_NARROW_ST, ALL>(smem, abase, H, G, bbase, token_ids, pair_gates, tiles, meta, act, y, act_ld);
   else
-    gemm_v3_body<MODE, 128, GP_STAGES>(smem, abase, H, G, bbase, token_ids, pair_gates, tiles, meta, act, y);
+    gemm_v3_body<MODE, 128, GP_STAGES, ALL>(smem, abase, H, G, bbase, token_ids, pair_gates, tiles, meta, act, y, act_ld);
 }
 
 // ------------------------------------------------------------------ short tiles
@@ -754,54 +773,11 @@ __global__ __launch_bounds__(GM_THREADS, 1) void gemm_s_kernel(
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// ------------------------------------------------------------------ combine
-// Per (token, 8 columns): the token's pair ids are read first (one batch of independent
-// loads), then up to CB_BATCH y rows at once, summed in expert order: two memory round
-// trips per batch instead of two per pair.
-#define CB_BATCH 8
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ y,
                                                       const int32_t* __restrict__ token_pairs,
                                                       const int32_t* __restrict__ count, int64_t N, int H,
                                                       int E, bf16_t* __restrict__ out) {
-  const int HC = H >> 3;
-  const int64_t total = N * HC;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t t = i / HC;
-    const int ch = (int)(i % HC);
-    float4 s0 = make_float4(0.f, 0.f, 0.f, 0.f), s1 = s0;
-    const int k = min(count[t], E);
-    const int32_t* tp = token_pairs + t * E;
-    bool stop = false;
-    for (int q0 = 0; q0 < k && !stop; q0 += CB_BATCH) {
-      int p[CB_BATCH];
-#pragma unroll
-      for (int i2 = 0; i2 < CB_BATCH; ++i2) p[i2] = q0 + i2 < k ? tp[q0 + i2] : -1;
-      float4 a[CB_BATCH], b[CB_BATCH];
-#pragma unroll
-      for (int i2 = 0; i2 < CB_BATCH; ++i2) {
-        // a negative id (fewer pairs than count: inconsistent caller data) ends the sum;
-        // nothing is read out of range
-        if (p[i2] >= 0) {
-          const float4* src = (const float4*)(y + (int64_t)p[i2] * H + ch * 8);
-          a[i2] = src[0];
-          b[i2] = src[1];
-        }
-      }
-#pragma unroll
-      for (int i2 = 0; i2 < CB_BATCH; ++i2) {
-        if (q0 + i2 >= k) break;
-        if (p[i2] < 0) { stop = true; break; }
-        s0.x += a[i2].x; s0.y += a[i2].y; s0.z += a[i2].z; s0.w += a[i2].w;
-        s1.x += b[i2].x; s1.y += b[i2].y; s1.z += b[i2].z; s1.w += b[i2].w;
-      }
-    }
-    uint4 o;
-    o.x = (uint32_t)f32_to_bf16(s0.x) | ((uint32_t)f32_to_bf16(s0.y) << 16);
-    o.y = (uint32_t)f32_to_bf16(s0.z) | ((uint32_t)f32_to_bf16(s0.w) << 16);
-    o.z = (uint32_t)f32_to_bf16(s1.x) | ((uint32_t)f32_to_bf16(s1.y) << 16);
-    o.w = (uint32_t)f32_to_bf16(s1.z) | ((uint32_t)f32_to_bf16(s1.w) << 16);
-    *(uint4*)(out + t * H + ch * 8) = o;
-  }
+  combine_rows<256, 1>(y, token_pairs, count, N, H, E, out);
 }
 
 // ------------------------------------------------------------------ host side
@@ -843,8 +819,8 @@ static void gemm_split_ptrs(void* gws, uint32_t** sync, float** part) {
 
 static int gateup_launch(const bf16_t* xb, int H, int G, const bf16_t* wrows, int E, const int32_t* token_ids,
                          const float* pair_gates, const int32_t* tiles, const int32_t* meta, int64_t max_tiles,
-                         bf16_t* act, void* gws, hipStream_t st, bool short_tiles = false) {
-  (void)E;
+                         bf16_t* act, void* gws, hipStream_t st, bool short_tiles = false,
+                         int min_pairs = INT_MAX) {
   uint32_t* sync;
   float* part;
   gemm_split_ptrs(gws, &sync, &part);
@@ -852,10 +828,17 @@ static int gateup_launch(const bf16_t* xb, int H, int G, const bf16_t* wrows, in
     gemm_s_kernel<0><<<gemm_s_grid(), GM_THREADS, GS_LDS_BYTES, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles,
                                                                       meta, act, nullptr, part, sync);
   } else if (G % 64 == 0) {
-    int grid = gemm_grid_v3(max_tiles * (G / 32));
-    constexpr int lds = std::max(Gv<0, 128, GP_STAGES>::LDS, Gv<0, 64, GP_NARROW_ST>::LDS);
-    gemm_v3_kernel<0><<<grid, GM_THREADS, lds, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles, meta, act, nullptr,
-                                                     pp_device_cus());
+    const int cus = pp_device_cus();
+    constexpr int wide = Gv<0, 128, GP_STAGES>::LDS, both = std::max(wide, Gv<0, 64, GP_NARROW_ST>::LDS);
+#define PP_GU(NARROW, ALL, NB, LDS)                                                                         \
+  gemm_v3_kernel<0, NARROW, ALL><<<gemm_grid_v3(max_tiles * (G / NB)), GM_THREADS, LDS, st>>>(                \
+      xb, H, G, wrows, token_ids, pair_gates, tiles, meta, act, nullptr, cus, min_pairs, E * G)
+    // the tile map's bound is E * N / 128 tiles: over 4 wide items per CU of it, a fraction of the
+    // experts selected still gives every CU one
+    if (min_pairs != INT_MAX) PP_GU(false, true, 64, wide);
+    else if (max_tiles * (G / 64) <= 4 * cus) PP_GU(true, false, 32, both);
+    else PP_GU(false, false, 64, wide);
+#undef PP_GU
   } else {
     int grid = gemm_grid(max_tiles * (G / 32));
     gateup_kernel<4, 1, 1><<<grid, GM_THREADS, 0, st>>>(xb, H, G, wrows, token_ids, pair_gates, tiles, meta, act);
@@ -865,7 +848,7 @@ static int gateup_launch(const bf16_t* xb, int H, int G, const bf16_t* wrows, in
 
 static int down_launch(const bf16_t* act, int H, int G, const bf16_t* down_t, const int32_t* tiles,
                        const int32_t* meta, int64_t max_tiles, float* y, void* gws, hipStream_t st,
-                       bool short_tiles = false) {
+                       bool short_tiles = false, int min_pairs = INT_MAX) {
   uint32_t* sync;
   float* part;
   gemm_split_ptrs(gws, &sync, &part);
@@ -873,9 +856,14 @@ static int down_launch(const bf16_t* act, int H, int G, const bf16_t* down_t, co
     gemm_s_kernel<1><<<gemm_s_grid(), GM_THREADS, GS_LDS_BYTES, st>>>(act, H, G, down_t, nullptr, nullptr, tiles,
                                                                       meta, nullptr, y, part, sync);
   } else if (G % 64 == 0) {
-    int grid = gemm_grid_v3(max_tiles * (H / 128));
-    gemm_v3_kernel<1><<<grid, GM_THREADS, Gv<1, 128, GP_STAGES>::LDS, st>>>(act, H, G, down_t, nullptr, nullptr, tiles,
-                                                                            meta, nullptr, y, 0);
+    const int grid = gemm_grid_v3(max_tiles * (H / 128));
+    constexpr int lds = Gv<1, 128, GP_STAGES>::LDS;
+    if (min_pairs != INT_MAX)
+      gemm_v3_kernel<1, false, true><<<grid, GM_THREADS, lds, st>>>(act, H, G, down_t, nullptr, nullptr, tiles, meta,
+                                                                    nullptr, y, 0, min_pairs, 0);
+    else
+      gemm_v3_kernel<1, false, false><<<grid, GM_THREADS, lds, st>>>(act, H, G, down_t, nullptr, nullptr, tiles, meta,
+                                                                     nullptr, y, 0, 0, 0);
   } else {
     int grid = gemm_grid(max_tiles * (H / 128));
     down_kernel<<<grid, GM_THREADS, 0, st>>>(act, H, G, down_t, tiles, meta, y);
@@ -935,19 +923,49 @@ int pp_route_impl(const void* x, int x_dtype, const float* logits_in, int64_t N,
 int pp_bucket_from_counts(const uint8_t* mask, const float* gates, int64_t N, int E, int tile_m,
                           const int32_t* blkcnt, int cb, int32_t* offsets, int32_t* token_ids, float* pair_gates,
                           int32_t* token_pairs, int32_t* tiles, int32_t* meta, hipStream_t st, uint32_t* zero,
-                          int nzero);
+                          int nzero, bf16_t* act, int G_act, int min_pairs);
 bool pp_bucket_counts_fit(int64_t N, int E, int cb);
 int pp_route_count_block(int64_t N, int H, int E);
 int pp_bucket_impl(const uint8_t* mask, const float* gates, int64_t N, int E, int tile_m, int32_t* offsets,
                    int32_t* token_ids, float* pair_gates, int32_t* token_pairs, int32_t* tiles, int32_t* meta,
                    void* workspace, hipStream_t st, uint32_t* zero, int nzero);
 
+size_t pp_dense_split_bytes();
+int pp_dense_split_words();
+int pp_dense_down(const bf16_t* act, int64_t n, int H, int E, int G, const bf16_t* down_t, bf16_t* out,
+                  uint32_t* sync, float* part, const int32_t* meta, int min_pairs, const uint8_t* mask,
+                  const float* y, const int32_t* token_pairs, const int32_t* count, hipStream_t st);
+
 struct PrefillWs {
   size_t gates, mask, count, offsets, token_ids, pair_gates, token_pairs, tiles, meta, bws, blk16, xbf, act, y,
-      gws, logits, total;
+      gws, logits, all_sync, all_part, total;
 };
 
-static PrefillWs prefill_layout(int64_t N, int H, int E, int G) {
+// Down projection over every expert at once. Grouped, a pair's down product is an fp32 row of H
+// written and read back (8191 tokens at tau 0.95, 13 of 16 experts each: down 248 us, combine 132);
+// as one [n][I] x [I][H] product of acts that are 0 for the experts a token does not select
+// (dense_gemm_kernel<1>, 154 us there) it has no such rows, and its time does not depend on the
+// selection. Which of the two is faster is known on the device, from the number of pairs P: the
+// product's launch does the combine instead below all_min_pairs, and the grouped down launch
+// nothing from there on. That choice costs the grouped side 2 % (one 512-thread workgroup per CU
+// combines, not five of 256), so it is offered where it is likely to be taken, from tau
+// PF_ALL_TAU on (16 experts with logits of std 0.8: 70 % of the pairs), and to calls longer than
+// a grouped pass: y is then sized for the grouped side's P alone, more tokens fit a pass, and one
+// pass less is worth more. Layer, us, before and now, E = 16, G = 384, H = 1536:
+//   tokens   tau 0.5        0.7        0.8        0.95
+//   2048                                        184 -> 167
+//   4096                                        340 -> 270
+//   5461     190 -> 162  271 -> 246  336 -> 299  511 -> 351
+//   8191     235 -> 222  380 -> 349  478 -> 365  714 -> 459
+// The line: at 4096 tokens the grouped side is faster at 38 % of the pairs (198 against 212 us),
+// the product at 52 % (237 against 250); at 2048 and 3072, where the product is cut into K ranges
+// and joined, at 52 % (140 / 153, 187 / 202) and 80 % (188 / 170, 267 / 243).
+#define PF_ALL_MIN 2048
+#define PF_ALL_TAU 0.9f
+#define PF_ALL_PCT(n) ((n) < 4096 ? 65 : 45)
+static int all_min_pairs(int64_t n, int E) { return (int)(n * E * PF_ALL_PCT(n) / 100); }
+
+static PrefillWs prefill_layout(int64_t N, int H, int E, int G, bool all = false) {
   PrefillWs L;
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -970,9 +988,11 @@ static PrefillWs prefill_layout(int64_t N, int H, int E, int G) {
   L.blk16 = take((size_t)((N + 3) / 4) * 16 * 4);  // the E = 16 router's per-block expert counts (>= 4 tokens a block)
   L.xbf = take((size_t)N * H * 2);
   L.act = take((size_t)P * G * 2);
-  L.y = take((size_t)P * H * 4);
+  L.y = take((size_t)(all ? all_min_pairs(N, E) : P) * H * 4);
   L.gws = prefill_short_tiles(N, H, G) ? take(gemm_split_bytes()) : 0;
   L.logits = E != 16 ? take((size_t)P * 4) : 0;  // the logits pass of E != 16 (selection from its logits)
+  L.all_sync = all ? take((size_t)pp_dense_split_words() * 4) : 0;
+  L.all_part = all ? take(pp_dense_split_bytes()) : 0;
   L.total = o;
   return L;
 }
@@ -988,6 +1008,23 @@ static int64_t prefill_pass_tokens(int64_t N, int H, int E) {
   const int64_t per_token = (int64_t)E * H * 4;
   // a multiple of 4 tokens: every pass's mask rows start 4-byte aligned (the bucketing reads words)
   return min(N, max((int64_t)64, PF_PASS_Y_BYTES / per_token / 4 * 4));
+}
+
+// Tokens per pass of the form with the down projection over every expert (0: not for this call).
+// Its y holds the pairs of the grouped case only, so more tokens fit the workspace of N (whose
+// size does not depend on the form); passes of equal length.
+static int64_t all_pass_tokens(int64_t N, int H, int E, int G, float tau) {
+  const int64_t ng = prefill_pass_tokens(N, H, E);
+  if (E != 16 || N < PF_ALL_MIN || (N <= ng && !(tau >= PF_ALL_TAU))) return 0;
+  const size_t have = prefill_layout(ng, H, E, G).total;
+  auto fits = [&](int64_t n) {
+    return pp_bucket_counts_fit(n, E, pp_route_count_block(n, H, E)) && prefill_layout(n, H, E, G, true).total <= have;
+  };
+  for (int64_t k = 1; N / k >= PF_ALL_MIN; ++k) {
+    const int64_t n = ((N + k - 1) / k + 3) / 4 * 4;  // (mask rows of every pass 4-byte aligned)
+    if (fits(n)) return N - (k - 1) * n >= 1 ? n : 0;
+  }
+  return 0;
 }
 
 size_t pp_dense_workspace_bytes(int64_t N, int H, int E, int G);
@@ -1007,9 +1044,9 @@ extern "C" size_t pp_prefill_workspace_bytes(int64_t n_tokens, int H, int E, int
 // One pass over n_tokens tokens (at most prefill_pass_tokens) on the workspace.
 static int prefill_pass(const void* x, int x_dtype, int64_t n_tokens, int H, const float* router_packed,
                         const float* bias, int E, int G, float tau, const void* packed, void* out_bf16,
-                        void* workspace, hipStream_t st, float* logits_out, uint8_t* mask_out) {
+                        void* workspace, hipStream_t st, float* logits_out, uint8_t* mask_out, bool all) {
   int rc;
-  const PrefillWs L = prefill_layout(n_tokens, H, E, G);
+  const PrefillWs L = prefill_layout(n_tokens, H, E, G, all);
   char* ws = (char*)workspace;
   float* gates = (float*)(ws + L.gates);
   uint8_t* mask = mask_out ? mask_out : (uint8_t*)(ws + L.mask);
@@ -1028,7 +1065,9 @@ static int prefill_pass(const void* x, int x_dtype, int64_t n_tokens, int H, con
   const int64_t mt = pp_max_tiles(n_tokens, E, tile_m);
   // the GEMMs' split workspace: its sync words are cleared by this call's bucketing kernel
   void* gws = short_tiles ? (void*)(ws + L.gws) : nullptr;
-  const int nzero = gws ? (int)(1 + gemm_split_slots()) : 0;
+  const int nzero = gws ? (int)(1 + gemm_split_slots()) : all ? pp_dense_split_words() : 0;
+  const int min_pairs = all ? all_min_pairs(n_tokens, E) : INT_MAX;
+  uint32_t* zero = gws ? (uint32_t*)gws : all ? (uint32_t*)(ws + L.all_sync) : nullptr;
   // E = 16: the router kernel also counts selections per 16-token block, and the
   // bucketing is one kernel from those counts (no counting or scan pass)
   const int cb = pp_route_count_block(n_tokens, H, E);
@@ -1039,16 +1078,19 @@ static int prefill_pass(const void* x, int x_dtype, int64_t n_tokens, int H, con
     return rc;
   if (blk16)
     rc = pp_bucket_from_counts(mask, gates, n_tokens, E, tile_m, blk16, cb, offsets, token_ids, pair_gates,
-                               token_pairs, tiles, meta, st, (uint32_t*)gws, nzero);
+                               token_pairs, tiles, meta, st, zero, nzero, all ? act : nullptr, G, min_pairs);
   else
     rc = pp_bucket_impl(mask, gates, n_tokens, E, tile_m, offsets, token_ids, pair_gates, token_pairs, tiles, meta,
                         ws + L.bws, st, (uint32_t*)gws, nzero);
   if (rc) return rc;
   if ((rc = gateup_launch(xbf, H, G, (const bf16_t*)packed, E, token_ids, pair_gates, tiles, meta, mt, act, gws,
-                          st, short_tiles)))
+                          st, short_tiles, min_pairs)))
     return rc;
   const bf16_t* down_t = (const bf16_t*)packed + (int64_t)E * G * 3 * H;
-  if ((rc = down_launch(act, H, G, down_t, tiles, meta, mt, y, gws, st, short_tiles))) return rc;
+  if ((rc = down_launch(act, H, G, down_t, tiles, meta, mt, y, gws, st, short_tiles, min_pairs))) return rc;
+  if (all)  // that product or, below min_pairs, the combine
+    return pp_dense_down(act, n_tokens, H, E, G, down_t, (bf16_t*)out_bf16, (uint32_t*)(ws + L.all_sync),
+                         (float*)(ws + L.all_part), meta, min_pairs, mask, y, token_pairs, count, st);
   return combine_launch(y, token_pairs, count, n_tokens, H, E, (bf16_t*)out_bf16, st);
 }
 
@@ -1068,13 +1110,17 @@ extern "C" int pp_moe_prefill_routed(const void* x, int x_dtype, int64_t n_token
   if (prefill_dense_form(G))
     return pp_dense_prefill(x, x_dtype, n_tokens, H, router_packed, bias, E, G, tau, packed, out_bf16, workspace,
                             (hipStream_t)stream, logits_out, mask_out);
-  const int64_t nc = prefill_pass_tokens(n_tokens, H, E);
+  int64_t nc = prefill_pass_tokens(n_tokens, H, E);
+  const int64_t na = all_pass_tokens(n_tokens, H, E, G, tau);
+  const bool all = na > 0;
+  if (all) nc = na;
   const size_t xs = x_dtype == PP_DTYPE_BF16 ? 2 : 4;
   for (int64_t n0 = 0; n0 < n_tokens; n0 += nc) {
     const int64_t nt = min(nc, n_tokens - n0);
     if ((rc = prefill_pass((const char*)x + (size_t)n0 * H * xs, x_dtype, nt, H, router_packed, bias, E, G, tau,
                            packed, (bf16_t*)out_bf16 + (size_t)n0 * H, workspace, (hipStream_t)stream,
-                           logits_out ? logits_out + n0 * E : nullptr, mask_out ? mask_out + n0 * E : nullptr)))
+                           logits_out ? logits_out + n0 * E : nullptr, mask_out ? mask_out + n0 * E : nullptr,
+                           all)))
       return rc;
   }
   return PP_OK;

@@ -873,7 +873,8 @@ __global__ __launch_bounds__(BKT_THREADS) void bucket_place_kernel(
     const uint8_t* __restrict__ mask, const float* __restrict__ gates, int64_t N, int E,
     const int32_t* __restrict__ blkcnt, int cb, int nblk_c, int tile_m, int32_t* __restrict__ offsets,
     int32_t* __restrict__ token_ids, float* __restrict__ pair_gates, int32_t* __restrict__ token_pairs,
-    int32_t* __restrict__ tiles, int32_t* __restrict__ meta, uint32_t* __restrict__ zero, int nzero) {
+    int32_t* __restrict__ tiles, int32_t* __restrict__ meta, uint32_t* __restrict__ zero, int nzero,
+    bf16_t* __restrict__ act, int G_act, int min_pairs) {
   __shared__ int cnt_s[BKT_PLACE_INTS];
   __shared__ int part_tot[BKT_THREADS], part_pre[BKT_THREADS];
   __shared__ int base_s[PP_MAX_EXPERTS];
@@ -944,6 +945,17 @@ __global__ __launch_bounds__(BKT_THREADS) void bucket_place_kernel(
   if (!has_tokens) return;  // N == 0: only the offsets / tile map
   __syncthreads();         // base_s
   bucket_scatter_pairs(gates, N, E, base_s, token_ids, pair_gates, token_pairs, tokw, expw, g_first);
+  // acts [N][E * G_act] of the experts a token does not select (min_pairs pairs or more: the down
+  // projection reads all of them): a thread takes the same 16-byte chunks of every token's row
+  if (!act || off_s[E] < min_pairs) return;  // uniform
+  const int nt = nb / E, row = E * G_act;
+  for (int c = tid; c < row / 8; c += BKT_THREADS) {
+    const int e = c / (G_act / 8);
+    uint4* p = (uint4*)(act + t0 * row) + c;
+#pragma unroll 4
+    for (int l = 0; l < nt; ++l)
+      if (!((expw[l][e >> 6] >> (e & 63)) & 1ull)) p[(int64_t)l * (row / 8)] = make_uint4(0u, 0u, 0u, 0u);
+  }
 }
 
 extern "C" size_t pp_bucket_workspace_bytes(int64_t n_tokens, int E) {
@@ -971,12 +983,12 @@ static bool bucket_place_fits(int64_t nblk_c, int E) { return nblk_c * E <= BKT_
 int pp_bucket_from_counts(const uint8_t* mask, const float* gates, int64_t N, int E, int tile_m,
                           const int32_t* blkcnt, int cb, int32_t* offsets, int32_t* token_ids, float* pair_gates,
                           int32_t* token_pairs, int32_t* tiles, int32_t* meta, hipStream_t st, uint32_t* zero,
-                          int nzero) {
+                          int nzero, bf16_t* act, int G_act, int min_pairs) {
   const int64_t nblk_c = (N + cb - 1) / cb;
   const int64_t nblk = (N + BKT_TOK - 1) / BKT_TOK;
   bucket_place_kernel<<<(unsigned)(nblk > 0 ? nblk : 1), BKT_THREADS, 0, st>>>(
       mask, gates, N, E, blkcnt, cb, (int)nblk_c, tile_m, offsets, token_ids, pair_gates, token_pairs, tiles, meta,
-      zero, zero ? nzero : 0);
+      zero, zero ? nzero : 0, act, G_act, min_pairs);
   return pp_check_launch("pp_bucket");
 }
 
@@ -989,7 +1001,7 @@ int pp_bucket_impl(const uint8_t* mask, const float* gates, int64_t N, int E, in
   if (nblk > 0) bucket_count_kernel<<<(unsigned)nblk, BKT_THREADS, 0, st>>>(mask, N, E, blkcnt);
   if (bucket_place_fits(nblk, E))
     return pp_bucket_from_counts(mask, gates, N, E, tile_m, blkcnt, BKT_TOK, offsets, token_ids, pair_gates,
-                                 token_pairs, tiles, meta, st, zero, nzero);
+                                 token_pairs, tiles, meta, st, zero, nzero, nullptr, 0, 0);
   bucket_scan_kernel<<<1, 256, 0, st>>>(blkcnt, (int)nblk, E, tile_m, blkoff, offsets, tiles, meta, zero,
                                         zero ? nzero : 0);
   if (nblk > 0)
