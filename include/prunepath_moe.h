@@ -256,7 +256,7 @@ int pp_moe_decode_batch(const void* x, int x_dtype, int64_t n_tokens, int H, con
  *     (token, expert): a token routes the same way in any batch) -> selection -> dense
  *     gate/up GEMM over every (token, neuron) with act = bf16(silu(g) * u * gate), 0 for the
  *     experts a token does not select -> dense down GEMM over all neurons, fp32
- *     accumulation, one rounding to bf16. Up to 256 tokens (64 above H = 1536): the same
+ *     accumulation, one rounding to bf16. Up to 224 tokens (64 above H = 1536): the same
  *     arithmetic in three launches that stream the weights. Passes of up to ~256 MiB of
  *     per-token buffers (about 15000 tokens at H = 1536, E = 192, G = 32).
  * Either way every token's routing is the same as in one pass over all N (its sums may be

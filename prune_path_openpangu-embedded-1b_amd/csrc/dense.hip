@@ -814,7 +814,7 @@ int pp_route_impl(const void* x, int x_dtype, const float* logits_in, int64_t N,
 // remaining column tiles as 128 x 256 tiles (three stages; a tail of those is K-split),
 // so that no 256-row tile is cut (at N = 2048, I = 6144: 256 + 256 tiles, one round each).
 // down: 256 x 192, K blocks of 64, two stages, waves 4 x 2 (wave tile 64 x 96), K-split
-// (at N = 2048, H = 1536: 64 tiles in four K ranges).
+// (at N = 2048, H = 1536: 64 tiles in four K ranges); 128-row tiles by down_short_tiles.
 #ifndef DG_GU_BM
 #define DG_GU_BM 256
 #endif
@@ -881,6 +881,9 @@ int pp_route_impl(const void* x, int x_dtype, const float* logits_in, int64_t N,
 #ifndef DG_DN_WPC
 #define DG_DN_WPC 1
 #endif
+// down of few row tiles: 128 x 192, three stages, waves 4 x 2 (wave tile 32 x 96)
+#define DG_DS_BM 128
+#define DG_DS_ST 3
 #define DG_SYNC_WORDS (4 * DG_MAX_GRID)   // per GEMM launch: 2 counters per tail item
 // one part's fp32 partial sums: a tile of either K-split launch (gate/up tail, down)
 #define DG_SLOT_BYTES                                                                                  \
@@ -958,9 +961,9 @@ static FewWs few_layout(int64_t n, int H, int I) {
   return L;
 }
 
-// Layers of 17.4 MB (E = 192, G = 32, H = 1536; us, GEMM tiles -> this form): 83 -> 27 at 2
-// tokens, 82 -> 28.7 at 16, 84 -> 37.7 at 64, 84 -> 49 at 128, 88 -> 72 at 256, where each token
-// block still costs 2.9 us in all and the GEMM tiles' time has not begun to grow. H > 1536: the
+// E = 192, G = 32, H = 1536, layer, us, GEMM tiles and this form: 83 / 27 at 2 tokens, 82 / 28.7 at
+// 16, 84 / 37.7 at 64, 67.6 / 49.5 at 128 (128-row down tiles), 69.0 / 61.4 at 192, 70.3 / 67.1 at
+// 224, 70.7 / 72.9 at 256; at H = 512 53.4 / 51.1 at 200, 54.9 / 57.7 at 256. H > 1536: the
 // weights no longer stay in registers over more than 64 tokens (H = 4096: 107 -> 84 at 64, 123 ->
 // 124 at 128). Buffers in the GEMMs' split workspace, which such a pass does not use.
 static bool dense_few_form(int64_t n, int H, int E, int G) {
@@ -978,6 +981,32 @@ static int dense_few_launch(const FewArgs& a, hipStream_t st) {
   if ((rc = pp_check_launch("dense_few_gateup_kernel"))) return rc;
   dense_few_down_kernel<DF_R, DF_KW><<<a.H / (16 * DF_R) * few_parts(a.I), 512, 0, st>>>(a);
   return pp_check_launch("dense_few_down_kernel");
+}
+
+// K blocks that the busiest workgroup of a launch walks over `tiles` tiles (GpSched's whole rounds
+// and tail parts).
+static int dense_blocks(int64_t tiles, int nkb) {
+  const int g = dense_grid();
+  const int64_t rounds = tiles / g;
+  const int tail = (int)(tiles - rounds * g);
+  if (tail == 0) return (int)(rounds * nkb);
+  const int parts = std::max(1, std::min(std::min(nkb / GP_MIN_PART_BLOCKS, g / tail), DG_NPMAX));
+  return (int)(rounds * nkb + (nkb + parts - 1) / parts);
+}
+
+// down: 128-row tiles where 256-row tiles would all be cut in K, unless the parts they can be cut
+// into leave them more than twice the K blocks. A block of theirs takes about half the time (three
+// stages in flight instead of two), their partial sums are half the bytes to join, and up to 128
+// tokens of padding go. E = 192, G = 32, H = 1536, layer, us, 256- and 128-row tiles: 84.2 / 67.9
+// at 257 tokens, 87.2 / 76.8 at 509, 123.7 / 116.1 at 1024, 286.5 / 275.3 at 4096; more than
+// twice the blocks: 153.2 / 154.7 at 1536, and 495 / 534 at E = 200, G = 160, H = 4096, 500 tokens.
+// Whole 256-row tiles stay: their operands cross L2 half as often (8191 tokens of the E = 16
+// prefill's product 466 / 505).
+static bool down_short_tiles(int64_t n, int H, int Ipad) {
+  const int64_t ct = (H + DG_DN_BN - 1) / DG_DN_BN;
+  const int64_t t256 = (n + DG_DN_BM - 1) / DG_DN_BM * ct, t128 = (n + DG_DS_BM - 1) / DG_DS_BM * ct;
+  const int nkb = Ipad / DG_DN_BK;
+  return 2 * t256 <= dense_grid() && dense_blocks(t128, nkb) <= 2 * dense_blocks(t256, nkb);
 }
 
 // One pass over n tokens (at most dense_pass_tokens). logits_out / mask_out (may be null)
@@ -1076,6 +1105,8 @@ static int dense_pass(const void* x, int x_dtype, int64_t n, int H, const float*
   a.out = out;
   a.ct_lo = 0;
   a.ct_hi = (H + DG_DN_BN - 1) / DG_DN_BN;
+  if (down_short_tiles(n, H, Ipad))
+    return dense_gemm_launch<1, DG_DS_BM, DG_DN_BN, DG_DN_BK, DG_DS_ST, DG_DN_NW, DG_DN_WR, DG_DN_WPC>(a, st);
   return dense_gemm_launch<1, DG_DN_BM, DG_DN_BN, DG_DN_BK, DG_DN_ST, DG_DN_NW, DG_DN_WR, DG_DN_WPC>(a, st);
 }
 

@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256, 1) void route_logits_few_kernel(const XT* __re
 }
 
 // ------------------------------------------------------------------ gate/up
-#define DF_MAX 256  // tokens at most
+#define DF_MAX 224  // tokens at most (dense_few_form)
 
 struct FewArgs {
   const bf16_t* xfrag;    // x as bf16: [H / 32][token block][lane][8]

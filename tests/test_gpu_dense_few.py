@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (1536, 192, 32, 15, torch.bfloat16),
     (1536, 192, 32, 16, torch.float32),
     (1536, 192, 32, 17, torch.bfloat16),
-    (1536, 192, 32, 256, torch.float32),   # the largest batch of the form
+    (1536, 192, 32, 224, torch.float32),   # the largest batch of the form
+    (1536, 192, 32, 225, torch.bfloat16),  # the first on GEMM tiles: 128-row down tiles in eight K parts
     (1536, 24, 32, 50, torch.bfloat16),    # selection in a launch of its own; 96 units in threes
     (1536, 5, 160, 33, torch.float32),     # 100 units: a last workgroup of one; five K steps an expert
     (1408, 65, 32, 70, torch.bfloat16),    # 44 K steps over eight waves; E just above the in-launch selection
@@ -26,6 +27,8 @@ pytestmark = pytest.mark.gpu
     (512, 200, 32, 129, torch.bfloat16),   # two groups of token blocks on weights loaded once
     (1664, 20, 96, 64, torch.float32),     # two K chunks, the second of one step
     (4096, 70, 32, 49, torch.bfloat16),    # three K chunks
+    (640, 5, 160, 300, torch.float32),     # down: a 128-row tile of 44 tokens, H in a short last column tile
+    (256, 70, 96, 1100, torch.bfloat16),   # nine 128-row tiles
 ])
 def test_dense_few_shapes(pkg, H, E, G, N, xdt):
     seed = H + E * 7 + G + N
