@@ -13,7 +13,9 @@
 //                          0 where the expert is not selected (never evaluated: no
 //                          inf * 0 from an unselected expert reaches the output)
 //   dense_gemm_kernel<1>   out[t, h] = bf16(sum over all neurons n of act[t, n] * Wd[n, h]),
-//                          fp32 accumulation, one rounding
+//                          fp32 accumulation, one rounding (also the E = 16 prefill's product
+//                          over every expert, with ALL: prefill.hip)
+// Small batches take the three kernels of dense_few.h instead.
 // Replaces moe_fused_expert_kernel (src/tl_kernel_optimized_Ultimate_PanGU.py:271-328) and
 // the TauSparseMoE.forward_prefill orchestration (:532-604) at these shapes, with the
 // reference's rounding points: bf16 act (acc_gate.to(bfloat16), :318-321) and fp32 sums

@@ -12,6 +12,8 @@
 //                  k-term combine -- enough to break atol 2e-3 on small outputs);
 //   combine_kernel out[t] = sum of y over the pairs of token t in expert order, fp32 ->
 //                  bf16 (deterministic, no atomics).
+// At E = 16 long calls with most pairs selected take one down product over every expert
+// (dense.hip) in place of the last two: all_pass_tokens, all_min_pairs.
 // Both GEMMs are persistent over a device-side tile map (no host sync, no padding FLOPs
 // beyond the last partial tile of each expert), 256 threads = 4 waves, BK = 64:
 // gemm_v3_kernel for G % 64 == 0 (LDS-DMA pipeline, below), gateup_kernel /
