@@ -964,8 +964,15 @@ struct PrefillWs {
 // and joined, at 52 % (140 / 153, 187 / 202) and 80 % (188 / 170, 267 / 243).
 #define PF_ALL_MIN 2048
 #define PF_ALL_TAU 0.9f
-#define PF_ALL_PCT(n) ((n) < 4096 ? 65 : 45)
-static int all_min_pairs(int64_t n, int E) { return (int)(n * E * PF_ALL_PCT(n) / 100); }
+// Wider experts have more products per y row: a pair's grouped time is taken as
+// proportional to 2.67 G + 1780 (its products at the grouped GEMM's rate, its row at the memory's), its
+// share of the whole product to 2 G, and the line above, measured at G = 384, moves with their
+// ratio; from there on no share of the pairs may reach it (G >= 2400), and the form is not offered.
+static int all_pct(int64_t n, int G) {
+  const double base = n < 4096 ? 65.0 : 45.0, w = G > 384 ? G : 384;
+  return (int)std::min(100.0, base * (w / (2.67 * w + 1780.0)) / (384.0 / (2.67 * 384.0 + 1780.0)));
+}
+static int all_min_pairs(int64_t n, int E, int G) { return (int)(n * E * all_pct(n, G) / 100); }
 
 static PrefillWs prefill_layout(int64_t N, int H, int E, int G, bool all = false) {
   PrefillWs L;
@@ -990,7 +997,7 @@ static PrefillWs prefill_layout(int64_t N, int H, int E, int G, bool all = false
   L.blk16 = take((size_t)((N + 3) / 4) * 16 * 4);  // the E = 16 router's per-block expert counts (>= 4 tokens a block)
   L.xbf = take((size_t)N * H * 2);
   L.act = take((size_t)P * G * 2);
-  L.y = take((size_t)(all ? all_min_pairs(N, E) : P) * H * 4);
+  L.y = take((size_t)(all ? all_min_pairs(N, E, G) : P) * H * 4);
   L.gws = prefill_short_tiles(N, H, G) ? take(gemm_split_bytes()) : 0;
   L.logits = E != 16 ? take((size_t)P * 4) : 0;  // the logits pass of E != 16 (selection from its logits)
   L.all_sync = all ? take((size_t)pp_dense_split_words() * 4) : 0;
@@ -1022,9 +1029,9 @@ static int64_t all_pass_tokens(int64_t N, int H, int E, int G, float tau) {
   auto fits = [&](int64_t n) {
     return pp_bucket_counts_fit(n, E, pp_route_count_block(n, H, E)) && prefill_layout(n, H, E, G, true).total <= have;
   };
-  for (int64_t k = 1; N / k >= PF_ALL_MIN; ++k) {
+  for (int64_t k = 1; k <= (N + ng - 1) / ng && N / k >= PF_ALL_MIN; ++k) {  // no more passes than grouped
     const int64_t n = ((N + k - 1) / k + 3) / 4 * 4;  // (mask rows of every pass 4-byte aligned)
-    if (fits(n)) return N - (k - 1) * n >= 1 ? n : 0;
+    if (all_pct(n, G) < 100 && fits(n)) return N - (k - 1) * n >= 1 ? n : 0;
   }
   return 0;
 }
@@ -1068,7 +1075,7 @@ static int prefill_pass(const void* x, int x_dtype, int64_t n_tokens, int H, con
   // the GEMMs' split workspace: its sync words are cleared by this call's bucketing kernel
   void* gws = short_tiles ? (void*)(ws + L.gws) : nullptr;
   const int nzero = gws ? (int)(1 + gemm_split_slots()) : all ? pp_dense_split_words() : 0;
-  const int min_pairs = all ? all_min_pairs(n_tokens, E) : INT_MAX;
+  const int min_pairs = all ? all_min_pairs(n_tokens, E, G) : INT_MAX;
   uint32_t* zero = gws ? (uint32_t*)gws : all ? (uint32_t*)(ws + L.all_sync) : nullptr;
   // E = 16: the router kernel also counts selections per 16-token block, and the
   // bucketing is one kernel from those counts (no counting or scan pass)

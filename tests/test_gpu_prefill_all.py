@@ -12,8 +12,12 @@ pytestmark = pytest.mark.gpu
 E, G, H = 16, 64, 256
 
 
-@pytest.mark.parametrize("N,tau", [(2048, 0.97), (3001, 0.3), (4096, 0.95), (4097, 0.3), (5003, 0.99), (9000, 0.97), (9000, 0.2)])
-def test_prefill_all_experts(pkg, N, tau):
+@pytest.mark.parametrize("H,N,tau", [
+    (H, 2048, 0.97), (H, 4096, 0.95), (H, 4097, 0.3), (H, 5003, 0.99),
+    (4096, 5000, 0.97), (4096, 5000, 0.2),  # longer than a grouped pass of 2048 tokens: two passes
+    (H, 9000, 0.97),                        # more tokens than the form's count table: grouped
+])
+def test_prefill_all_experts(pkg, H, N, tau):
     w = gi.layer_weights(N, H=H, I=E * G, E=E)
     m = make_module(pkg, w, tau)
     xg = to_gpu(gi.tokens(N + 1, N, H=H), torch.bfloat16 if N % 2 else torch.float32)
