@@ -967,7 +967,7 @@ struct PrefillWs {
 // Wider experts have more products per y row: a pair's grouped time is taken as
 // proportional to 2.67 G + 1780 (its products at the grouped GEMM's rate, its row at the memory's), its
 // share of the whole product to 2 G, and the line above, measured at G = 384, moves with their
-// ratio; from there on no share of the pairs may reach it (G >= 2400), and the form is not offered.
+// ratio; at 100 % (G >= 2944, below 4096 tokens G >= 896) the form is not offered.
 static int all_pct(int64_t n, int G) {
   const double base = n < 4096 ? 65.0 : 45.0, w = G > 384 ? G : 384;
   return (int)std::min(100.0, base * (w / (2.67 * w + 1780.0)) / (384.0 / (2.67 * 384.0 + 1780.0)));
