@@ -277,6 +277,14 @@ int pp_moe_prefill_routed(const void* x, int x_dtype, int64_t n_tokens, int H,
                           const void* packed, void* out_bf16, void* workspace,
                           float* logits_out, uint8_t* mask_out, void* stream);
 
+/* How pp_moe_prefill cuts such a call: returns its number of passes (0: arguments out of range
+ * or G % 64 != 0) and writes for pass `index`, each where not NULL, its tokens, the number of
+ * selected pairs from which it takes the down GEMM over every expert (-1: not offered), and the
+ * bytes of workspace it lays out, at most pp_prefill_workspace_bytes. Host arithmetic. No
+ * counterpart in the reference. */
+int64_t pp_prefill_pass(int64_t n_tokens, int H, int E, int G, float tau, int64_t index, int64_t* tokens,
+                        int64_t* min_pairs, size_t* workspace_bytes);
+
 /* Stages of pp_moe_prefill, exposed for testing and for callers that route
  * elsewhere. x is bf16 [N,H]. act is bf16 [N*E][G] capacity (row = pair), y is
  * fp32 [N*E][H] capacity (row = pair). */

@@ -63,6 +63,7 @@ SIGNATURES = {
                                c_void_p, c_void_p, c_void_p, c_void_p]),
     "pp_moe_prefill_routed": (c_int, [c_void_p, c_int, c_int64, c_int, c_void_p, c_void_p, c_int, c_int, c_float,
                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "pp_prefill_pass": (c_int64, [c_int64, c_int, c_int, c_int, c_float, c_int64, c_void_p, c_void_p, c_void_p]),
     "pp_expert_gateup": (c_int, [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_int64, c_void_p, c_void_p]),
     "pp_expert_down": (c_int, [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_int64,

@@ -972,9 +972,11 @@ static int all_pct(int64_t n, int G) {
   const double base = n < 4096 ? 65.0 : 45.0, w = G > 384 ? G : 384;
   return (int)std::min(100.0, base * (w / (2.67 * w + 1780.0)) / (384.0 / (2.67 * 384.0 + 1780.0)));
 }
-static int all_min_pairs(int64_t n, int E, int G) { return (int)(n * E * all_pct(n, G) / 100); }
+static int all_min_pairs(int64_t n, int E, int pct) { return (int)(n * E * pct / 100); }
 
-static PrefillWs prefill_layout(int64_t N, int H, int E, int G, bool all = false) {
+// pct: the call's share of the pairs from which the product is taken, 0 where it is not offered.
+static PrefillWs prefill_layout(int64_t N, int H, int E, int G, int pct) {
+  const bool all = pct > 0;
   PrefillWs L;
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -997,7 +999,7 @@ static PrefillWs prefill_layout(int64_t N, int H, int E, int G, bool all = false
   L.blk16 = take((size_t)((N + 3) / 4) * 16 * 4);  // the E = 16 router's per-block expert counts (>= 4 tokens a block)
   L.xbf = take((size_t)N * H * 2);
   L.act = take((size_t)P * G * 2);
-  L.y = take((size_t)(all ? all_min_pairs(N, E, G) : P) * H * 4);
+  L.y = take((size_t)(all ? all_min_pairs(N, E, pct) : P) * H * 4);
   L.gws = prefill_short_tiles(N, H, G) ? take(gemm_split_bytes()) : 0;
   L.logits = E != 16 ? take((size_t)P * 4) : 0;  // the logits pass of E != 16 (selection from its logits)
   L.all_sync = all ? take((size_t)pp_dense_split_words() * 4) : 0;
@@ -1019,21 +1021,33 @@ static int64_t prefill_pass_tokens(int64_t N, int H, int E) {
   return min(N, max((int64_t)64, PF_PASS_Y_BYTES / per_token / 4 * 4));
 }
 
-// Tokens per pass of the form with the down projection over every expert (0: not for this call).
-// Its y holds the pairs of the grouped case only, so more tokens fit the workspace of N (whose
-// size does not depend on the form); passes of equal length.
-static int64_t all_pass_tokens(int64_t N, int H, int E, int G, float tau) {
+// What a call's passes share: their length (the last one takes what is left) and pct, 0 for the
+// grouped form. With the down projection over every expert offered, y holds the pairs of the
+// grouped case only, so more tokens fit the workspace of N (whose size does not depend on the
+// form); passes of equal length. pct is the first pass's for all of them: the share is larger for
+// shorter passes, and a shorter last pass with a share of its own would need a larger y than the
+// first. The last pass is checked by itself all the same.
+struct PrefillPlan {
+  int64_t tokens;
+  int pct;
+};
+static PrefillPlan prefill_plan(int64_t N, int H, int E, int G, float tau) {
   const int64_t ng = prefill_pass_tokens(N, H, E);
-  if (E != 16 || N < PF_ALL_MIN || (N <= ng && !(tau >= PF_ALL_TAU))) return 0;
-  const size_t have = prefill_layout(ng, H, E, G).total;
-  auto fits = [&](int64_t n) {
-    return pp_bucket_counts_fit(n, E, pp_route_count_block(n, H, E)) && prefill_layout(n, H, E, G, true).total <= have;
+  const PrefillPlan grouped = {ng, 0};
+  if (E != 16 || N < PF_ALL_MIN || (N <= ng && !(tau >= PF_ALL_TAU))) return grouped;
+  const size_t have = prefill_layout(ng, H, E, G, 0).total;
+  auto fits = [&](int64_t n, int pct) {
+    // (the product's bucketing clears the product's counters, short tiles their own)
+    return n > 0 && !prefill_short_tiles(n, H, G) && pp_bucket_counts_fit(n, E, pp_route_count_block(n, H, E)) &&
+           prefill_layout(n, H, E, G, pct).total <= have;
   };
   for (int64_t k = 1; k <= (N + ng - 1) / ng && N / k >= PF_ALL_MIN; ++k) {  // no more passes than grouped
     const int64_t n = ((N + k - 1) / k + 3) / 4 * 4;  // (mask rows of every pass 4-byte aligned)
-    if (all_pct(n, G) < 100 && fits(n)) return N - (k - 1) * n >= 1 ? n : 0;
+    const int64_t first = min(n, N);
+    const int pct = all_pct(first, G);
+    if (pct < 100 && fits(first, pct) && fits(N - (k - 1) * n, pct)) return {n, pct};
   }
-  return 0;
+  return grouped;
 }
 
 size_t pp_dense_workspace_bytes(int64_t N, int H, int E, int G);
@@ -1047,15 +1061,35 @@ static bool prefill_dense_form(int G) { return G % 64 != 0; }
 
 extern "C" size_t pp_prefill_workspace_bytes(int64_t n_tokens, int H, int E, int G) {
   if (prefill_dense_form(G)) return pp_dense_workspace_bytes(n_tokens, H, E, G);
-  return prefill_layout(prefill_pass_tokens(n_tokens, H, E), H, E, G).total;
+  return prefill_layout(prefill_pass_tokens(n_tokens, H, E), H, E, G, 0).total;
 }
 
-// One pass over n_tokens tokens (at most prefill_pass_tokens) on the workspace.
+extern "C" int64_t pp_prefill_pass(int64_t n_tokens, int H, int E, int G, float tau, int64_t index, int64_t* tokens,
+                                   int64_t* min_pairs, size_t* workspace_bytes) {
+  if (pp_check_shape(H, E, G) || n_tokens <= 0 || n_tokens > (int64_t)0x7fffffff / PP_MAX_EXPERTS ||
+      prefill_dense_form(G))
+    return 0;
+  const PrefillPlan plan = prefill_plan(n_tokens, H, E, G, tau);
+  const int64_t passes = (n_tokens + plan.tokens - 1) / plan.tokens;
+  if (index >= 0 && index < passes) {
+    const int64_t nt = min(plan.tokens, n_tokens - index * plan.tokens);
+    if (tokens) *tokens = nt;
+    if (min_pairs) *min_pairs = plan.pct ? all_min_pairs(nt, E, plan.pct) : -1;
+    if (workspace_bytes) *workspace_bytes = prefill_layout(nt, H, E, G, plan.pct).total;
+  }
+  return passes;
+}
+
+// One pass over n_tokens tokens on the workspace (ws_bytes of it), with the call's pct (prefill_plan).
 static int prefill_pass(const void* x, int x_dtype, int64_t n_tokens, int H, const float* router_packed,
                         const float* bias, int E, int G, float tau, const void* packed, void* out_bf16,
-                        void* workspace, hipStream_t st, float* logits_out, uint8_t* mask_out, bool all) {
+                        void* workspace, size_t ws_bytes, hipStream_t st, float* logits_out, uint8_t* mask_out,
+                        int pct) {
   int rc;
-  const PrefillWs L = prefill_layout(n_tokens, H, E, G, all);
+  const bool all = pct > 0;
+  const PrefillWs L = prefill_layout(n_tokens, H, E, G, pct);
+  PP_REQUIRE(L.total <= ws_bytes, PP_ERR_INVALID, "pp_moe_prefill: a pass of %lld tokens needs %zu of %zu bytes",
+             (long long)n_tokens, L.total, ws_bytes);
   char* ws = (char*)workspace;
   float* gates = (float*)(ws + L.gates);
   uint8_t* mask = mask_out ? mask_out : (uint8_t*)(ws + L.mask);
@@ -1075,7 +1109,7 @@ static int prefill_pass(const void* x, int x_dtype, int64_t n_tokens, int H, con
   // the GEMMs' split workspace: its sync words are cleared by this call's bucketing kernel
   void* gws = short_tiles ? (void*)(ws + L.gws) : nullptr;
   const int nzero = gws ? (int)(1 + gemm_split_slots()) : all ? pp_dense_split_words() : 0;
-  const int min_pairs = all ? all_min_pairs(n_tokens, E, G) : INT_MAX;
+  const int min_pairs = all ? all_min_pairs(n_tokens, E, pct) : INT_MAX;
   uint32_t* zero = gws ? (uint32_t*)gws : all ? (uint32_t*)(ws + L.all_sync) : nullptr;
   // E = 16: the router kernel also counts selections per 16-token block, and the
   // bucketing is one kernel from those counts (no counting or scan pass)
@@ -1119,17 +1153,16 @@ extern "C" int pp_moe_prefill_routed(const void* x, int x_dtype, int64_t n_token
   if (prefill_dense_form(G))
     return pp_dense_prefill(x, x_dtype, n_tokens, H, router_packed, bias, E, G, tau, packed, out_bf16, workspace,
                             (hipStream_t)stream, logits_out, mask_out);
-  int64_t nc = prefill_pass_tokens(n_tokens, H, E);
-  const int64_t na = all_pass_tokens(n_tokens, H, E, G, tau);
-  const bool all = na > 0;
-  if (all) nc = na;
+  const PrefillPlan plan = prefill_plan(n_tokens, H, E, G, tau);
+  const int64_t nc = plan.tokens;
+  const size_t ws_bytes = pp_prefill_workspace_bytes(n_tokens, H, E, G);
   const size_t xs = x_dtype == PP_DTYPE_BF16 ? 2 : 4;
   for (int64_t n0 = 0; n0 < n_tokens; n0 += nc) {
     const int64_t nt = min(nc, n_tokens - n0);
     if ((rc = prefill_pass((const char*)x + (size_t)n0 * H * xs, x_dtype, nt, H, router_packed, bias, E, G, tau,
-                           packed, (bf16_t*)out_bf16 + (size_t)n0 * H, workspace, (hipStream_t)stream,
+                           packed, (bf16_t*)out_bf16 + (size_t)n0 * H, workspace, ws_bytes, (hipStream_t)stream,
                            logits_out ? logits_out + n0 * E : nullptr, mask_out ? mask_out + n0 * E : nullptr,
-                           all)))
+                           plan.pct)))
       return rc;
   }
   return PP_OK;

@@ -147,3 +147,16 @@ def abi_prefill(pkg, m, xs, E, G, tau=0.7, routed=True):
                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
                    "moe_prefill_routed")
     return y, lg, mk
+
+
+def prefill_passes(lib, N, H, E, G, tau, pick=None):
+    """[(tokens, min_pairs, workspace bytes)] of the passes of a grouped prefill call (those of
+    the indices ``pick``; all by default)."""
+    import ctypes
+    t, m, b = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_size_t()
+    n = lib.pp_prefill_pass(N, H, E, G, tau, -1, None, None, None)
+    out = []
+    for i in range(n) if pick is None else sorted(set(p % n for p in pick)):
+        assert lib.pp_prefill_pass(N, H, E, G, tau, i, ctypes.byref(t), ctypes.byref(m), ctypes.byref(b)) == n
+        out.append((t.value, m.value, b.value))
+    return out

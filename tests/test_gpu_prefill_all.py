@@ -15,6 +15,7 @@ E, G, H = 16, 64, 256
 @pytest.mark.parametrize("H,N,tau", [
     (H, 2048, 0.97), (H, 4096, 0.95), (H, 4097, 0.3), (H, 5003, 0.99),
     (4096, 5000, 0.97), (4096, 5000, 0.2),  # longer than a grouped pass of 2048 tokens: two passes
+    (3072, 8191, 0.95),                     # passes of 4096 and 4095 tokens, where the share changes
     (H, 9000, 0.97),                        # more tokens than the form's count table: grouped
 ])
 def test_prefill_all_experts(pkg, H, N, tau):
