@@ -149,6 +149,26 @@ __device__ __forceinline__ void dg_tile(int item, int n_rt, int n_ct, int gr, in
   rt = q * gr + (r - ctl * rows);
 }
 
+// ALL: output column h of token t over its selected experts alone (G % 64 == 0), for a sum that is
+// infinite or NaN: the other experts' acts are 0, and 0 times an infinite or NaN weight is NaN.
+__device__ __forceinline__ float dg_selected_sum(const DgArgs& p, int64_t t, int h) {
+  float s = 0.0f;
+  for (int e = 0; e < p.E; ++e) {
+    if (!p.mask[t * p.E + e]) continue;
+    const uint4* av = (const uint4*)(p.a + t * p.Ipad + e * p.G);
+    const uint4* wv = (const uint4*)(p.b + ((int64_t)e * p.H + h) * p.G);
+    float d = 0.0f;
+    for (int g = 0; g < p.G / 8; ++g) {
+      const bf16x8_t a = as_bf16x8(av[g]), b = as_bf16x8(wv[g]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) d = fmaf((float)a[i], (float)b[i], d);
+    }
+    s += d;
+  }
+  return s;
+}
+__device__ __forceinline__ bool dg_finite(float v) { return __builtin_fabsf(v) < __builtin_huge_valf(); }
+
 // ALL (MODE 1): the E = 16 prefill's launch, with the other uses of DgArgs::meta; a template
 // parameter, as the code alone cost the dense form's down launch 1 us.
 template <int MODE, int BM, int BN, int BK, int STAGES, int NW, int WR, int WPC, bool ALL>
@@ -183,7 +203,7 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
   const GpSched sc(n_items, nkb, p.sync != nullptr, DG_NPMAX);
   const int F = sc.units(nkb);
   if (F <= 0) return;
-  bool odd = false;  // ALL: a result of this thread is infinite or NaN
+  bool odd = false;  // ALL: a result of this thread in a whole tile is infinite or NaN
 
   // ---- DMA issue cursor. Wave w, instruction i covers tile rows (NW i + w) * RPI .. + RPI;
   // lane l takes row (NW i + w) * RPI + l / CH and LDS chunk position l % CH, i.e. global
@@ -458,8 +478,9 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
                 p.out[(t0 + rl) * p.Ipad + n] = f32_to_bf16(a);
               } else {
                 const int hc = ct * BN + wn * C::WC + col;
-                if (hc < p.H) p.out[(t0 + rl) * p.H + hc] = f32_to_bf16(sv[h]);
-                if (ALL) odd |= !(__builtin_fabsf(sv[h]) < __builtin_huge_valf());
+                if (hc >= p.H) continue;
+                if (ALL && !dg_finite(sv[h])) sv[h] = dg_selected_sum(p, t0 + rl, hc);
+                p.out[(t0 + rl) * p.H + hc] = f32_to_bf16(sv[h]);
               }
             }
           }
@@ -527,7 +548,7 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
                 for (int q = 0; q < 16; ++q) {
                   const int rl = i * 32 + mfma32_row(q, ln);
                   *(bf16_t*)(ep + (rl - hf * RP) * RW + (nl - jg * 32) * 2) = f32_to_bf16(v[q]);
-                  if (ALL) odd |= !(__builtin_fabsf(v[q]) < __builtin_huge_valf());
+                  if (ALL) odd |= !dg_finite(v[q]);
                 }
               }
             }
@@ -549,27 +570,17 @@ __global__ __launch_bounds__(NW * 64, WPC) void dense_gemm_kernel(DgArgs p) {
   // the redundant tail DMAs must land before the workgroup's LDS is released
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (ALL && __syncthreads_or(odd)) {
-    // Infinite or NaN results again, over the selected experts alone: the others' acts are 0, and 0
-    // times an infinite or NaN weight is NaN. Every element of the workgroup's tiles is looked at
-    // (of a split tile also those that other workgroups reduce: they do the same after their own
-    // stores, and write the same values).
-    for (int li = 0; li < n_local; ++li) {
+    // Infinite or NaN results of the workgroup's whole tiles again. A split tile's are dealt with
+    // where they are reduced, by the thread that stores them: its other elements belong to other
+    // workgroups, which may not have stored them yet.
+    for (int li = 0; li < sc.n_whole; ++li) {
       int ctl, rt;
       dg_tile(sc.item(li), n_rt, n_ct, DG_DN_GR, rt, ctl);
       for (int i = tid; i < BM * BN; i += C::NT) {
         const int64_t t = (int64_t)rt * BM + i / BN;
         const int h = (p.ct_lo + ctl) * BN + i % BN;
-        if (t >= p.N || h >= p.H || (p.out[t * p.H + h] & 0x7f80u) != 0x7f80u) continue;
-        float s = 0.0f;
-        for (int e = 0; e < p.E; ++e) {
-          if (!p.mask[t * p.E + e]) continue;
-          const bf16_t* av = p.a + t * p.Ipad + e * p.G;
-          const bf16_t* wv = p.b + ((int64_t)e * p.H + h) * p.G;
-          float d = 0.0f;
-          for (int g = 0; g < p.G; ++g) d = fmaf(bf16_to_f32(av[g]), bf16_to_f32(wv[g]), d);
-          s += d;
-        }
-        p.out[t * p.H + h] = f32_to_bf16(s);
+        if (t < p.N && h < p.H && (p.out[t * p.H + h] & 0x7f80u) == 0x7f80u)
+          p.out[t * p.H + h] = f32_to_bf16(dg_selected_sum(p, t, h));
       }
     }
   }

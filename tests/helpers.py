@@ -128,13 +128,15 @@ def assert_close(got: np.ndarray, ref: np.ndarray, rtol=RTOL, atol=ATOL, what=""
                              f"max abs err {err.max():.3e}")
 
 
-def abi_prefill(pkg, m, xs, E, G, tau=0.7, routed=True):
+def abi_prefill(pkg, m, xs, E, G, tau=0.7, routed=True, fill=None):
     """pp_moe_prefill_routed through the C ABI on the module's buffers: (out bf16 [n,H],
     logits fp32 [n,E], mask uint8 [n,E]) -- the routing the call itself used (routed=False:
-    no routing outputs requested)."""
+    no routing outputs requested; fill: what the output holds before the call)."""
     import ctypes
     n, H = xs.shape
     y = torch.empty(n, H, dtype=torch.bfloat16, device=xs.device)
+    if fill is not None:
+        y.fill_(fill)
     lg = torch.empty(n, E, dtype=torch.float32, device=xs.device)
     mk = torch.empty(n, E, dtype=torch.uint8, device=xs.device)
     ws = torch.empty(pkg.ops.prefill_workspace_bytes(n, H, E, G), dtype=torch.uint8, device=xs.device)

@@ -6,7 +6,8 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import abi_prefill, assert_close, dev, gi, make_module, oracle, sparse_expected_gpu, to_gpu
+from helpers import (abi_prefill, assert_close, dev, gi, make_module, oracle, prefill_passes, sparse_expected_gpu,
+                     to_gpu)
 
 pytestmark = pytest.mark.gpu
 E, G, H = 16, 64, 256
@@ -31,26 +32,46 @@ def test_prefill_all_experts(pkg, H, N, tau):
     assert torch.equal(y, y2)
 
 
+def offered(pkg, N, H, tau, mask, taken):
+    """The call's passes are offered the product and have the pairs for it (taken), or not."""
+    t0 = 0
+    for t, min_pairs, _ in prefill_passes(pkg._lib.lib(), N, H, E, G, tau):
+        assert min_pairs >= 0, "grouped form"
+        assert (int(mask[t0:t0 + t].sum()) >= min_pairs) == taken
+        t0 += t
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
-def test_prefill_all_experts_nonfinite_weights(pkg, bad):
-    N, tau = 4100, 0.9
+@pytest.mark.parametrize("H,N", [
+    (512, 4100),   # 17 x 3 tiles, all of them cut in K
+    (1664, 8192),  # 32 x 9 tiles: one round of whole tiles, the rest cut in K
+])
+def test_prefill_all_experts_nonfinite_weights(pkg, H, N, bad):
+    """The elements that a bad weight reaches, and the bits of all others, whatever the output held
+    before the call: a workgroup must not take what another has not stored yet for a result."""
+    tau = 0.95
     w = gi.layer_weights(3, H=H, I=E * G, E=E)
     xg = to_gpu(gi.tokens(4, N, H=H))
     m = make_module(pkg, w, tau)
     y, _, mk = abi_prefill(pkg, m, xg, E, G, tau=tau)
-    assert mk.float().mean() > 0.5  # the side under test
+    offered(pkg, N, H, tau, mk, True)
     perm = oracle.pack_permutation(w["expert_ids"])
     w2 = dict(w, w_down=w["w_down"].copy())
-    w2["w_down"][7, perm[5 * G + 3]] = bad  # expert 5, output column 7
-    y2, _, mk2 = abi_prefill(pkg, make_module(pkg, w2, tau), xg, E, G, tau=tau)
-    assert torch.equal(mk, mk2)
     hit = torch.zeros(N, H, dtype=torch.bool, device=dev())
-    hit[:, 7] = mk[:, 5].bool()
+    for e, g, h in [(5, 3, 7), (5, 40, H - 1), (15, 63, 200), (0, 0, 300)]:  # expert, neuron, output column
+        w2["w_down"][h, perm[e * G + g]] = bad
+        hit[:, h] = mk[:, e].bool()
+    m2 = make_module(pkg, w2, tau)
+    y2, _, mk2 = abi_prefill(pkg, m2, xg, E, G, tau=tau, fill=0.0)
+    assert torch.equal(mk, mk2)
     assert bool((~torch.isfinite(y2.float()))[hit].all())
     assert torch.equal(torch.isfinite(y2.float()), ~hit)
-    clean = ~hit
-    clean[:, 7] = False
-    assert torch.equal(y2[clean], y[clean])
-    rest = ~mk[:, 5].bool()  # column 7 again, summed over the selected experts alone
-    d = (y2[rest, 7].float() - y[rest, 7].float()).abs()
-    assert bool((d <= 2e-3 + 2e-2 * y[rest, 7].float().abs()).all())
+    cols = hit.any(0)
+    assert torch.equal(y2[:, ~cols], y[:, ~cols])
+    # the same columns, summed over the selected experts alone
+    rest = cols[None] & ~hit
+    d = (y2[rest].float() - y[rest].float()).abs()
+    assert bool((d <= 2e-3 + 2e-2 * y[rest].float().abs()).all())
+    for fill in (float("nan"), float("inf")):
+        y3, _, _ = abi_prefill(pkg, m2, xg, E, G, tau=tau, fill=fill)
+        assert torch.equal(y3.view(torch.int16), y2.view(torch.int16))
