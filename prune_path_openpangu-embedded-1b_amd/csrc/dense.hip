@@ -976,7 +976,7 @@ static FewWs few_layout(int64_t n, int H, int I) {
 
 // E = 192, G = 32, H = 1536, layer, us, GEMM tiles and this form: 83 / 27 at 2 tokens, 82 / 28.7 at
 // 16, 84 / 37.7 at 64, 67.6 / 49.5 at 128 (128-row down tiles), 69.0 / 61.4 at 192, 70.3 / 67.1 at
-// 224, 70.7 / 72.9 at 256; at H = 512 53.4 / 51.1 at 200, 54.9 / 57.7 at 256. H > 1536: the
+// 224, 70.7 / 72.9 at 256; at H = 512 53.4 / 45.7 at 200. H > 1536: the
 // weights no longer stay in registers over more than 64 tokens (H = 4096: 107 -> 84 at 64, 123 ->
 // 124 at 128). Buffers in the GEMMs' split workspace, which such a pass does not use.
 static bool dense_few_form(int64_t n, int H, int E, int G) {
@@ -987,10 +987,23 @@ static bool dense_few_form(int64_t n, int H, int E, int G) {
 static int dense_few_launch(const FewArgs& a, hipStream_t st) {
   int rc;
   const int units = a.I / 8;
-  if (a.H == 1536)  // six K steps a wave, all in registers
-    dense_few_gateup_kernel<3, 6, true><<<a.n_sel + (units + 2) / 3, 512, 0, st>>>(a);
-  else
-    dense_few_gateup_kernel<2, 6, false><<<a.n_sel + (units + 1) / 2, 512, 0, st>>>(a);
+  // H = 256 KS up to 1536: KS whole K steps a wave, weights in registers over all token blocks.
+  // Against the chunked form (the same bits), us a layer at E = 192, G = 32, 16 / 64 / 200 tokens:
+  // H = 256 14.8 / 22.1 / 48.8 -> 14.8 / 21.8 / 43.6, 512 16.8 / 25.2 / 50.5 -> 16.9 / 24.1 / 45.7,
+  // 768 19.1 / 27.8 / 52.2 -> 18.3 / 26.2 / 48.1, 1024 22.2 / 30.8 / 55.4 -> 20.9 / 28.5 / 51.5,
+  // 1280 27.1 / 37.1 / 65.1 -> 25.2 / 33.7 / 59.8. With a test for the wave's last step in the place
+  // of whole steps (any H up to 1536) H = 1536 takes 27.9 -> 30.0 at 16 tokens.
+#define DF_GU(U, KS, ONE) dense_few_gateup_kernel<U, KS, ONE><<<a.n_sel + (units + U - 1) / U, 512, 0, st>>>(a)
+  switch (a.H % 256 == 0 ? a.H / 256 : 0) {
+    case 1: DF_GU(3, 1, true); break;
+    case 2: DF_GU(3, 2, true); break;
+    case 3: DF_GU(3, 3, true); break;
+    case 4: DF_GU(3, 4, true); break;
+    case 5: DF_GU(3, 5, true); break;
+    case 6: DF_GU(3, 6, true); break;
+    default: DF_GU(2, 6, false);
+  }
+#undef DF_GU
   if ((rc = pp_check_launch("dense_few_gateup_kernel"))) return rc;
   dense_few_down_kernel<DF_R, DF_KW><<<a.H / (16 * DF_R) * few_parts(a.I), 512, 0, st>>>(a);
   return pp_check_launch("dense_few_down_kernel");

@@ -166,7 +166,7 @@ __device__ __forceinline__ int64_t few_h(int n, int tb, int tok, int ntb) {
 // them loaded at a time. The eight waves' partial sums are added in wave order through LDS.
 // ONE: every wave has exactly KS K steps (H = 256 KS), so the weights stay in registers over all
 // token blocks. U = 3 there: at I = 6144 one workgroup per CU (and the selection's beside them in
-// the 128 VGPRs that leave room for two), N = 16 / 64 / 128: 28.7 / 37.7 / 49.2 us a layer
+// the 128 VGPRs that leave room for two), H = 1536, N = 16 / 64 / 128: 28.7 / 37.7 / 49.2 us a layer
 // against 30.4 / 40.4 / 52.7 with U = 2 and 30.8 / 40.8 / 54.2 with U = 1. x in operand order
 // instead of token rows (each load 16 rows x 64 B): 46 -> 40 us at N = 64.
 template <int U, int KS, bool ONE>

@@ -24,7 +24,12 @@ pytestmark = pytest.mark.gpu
     (1536, 5, 160, 33, torch.float32),     # 100 units: a last workgroup of one; five K steps an expert
     (1408, 65, 32, 70, torch.bfloat16),    # 44 K steps over eight waves; E just above the in-launch selection
     (128, 3, 32, 100, torch.float32),      # four K steps, four waves without any
-    (512, 200, 32, 129, torch.bfloat16),   # two groups of token blocks on weights loaded once
+    (256, 66, 32, 40, torch.float32),      # one whole K step a wave
+    (512, 200, 32, 129, torch.bfloat16),   # two
+    (768, 24, 32, 16, torch.float32),      # three
+    (1024, 5, 160, 100, torch.bfloat16),   # four
+    (1280, 100, 32, 17, torch.float32),    # five
+    (640, 200, 32, 129, torch.bfloat16),   # two groups of token blocks on weights loaded once
     (1664, 20, 96, 64, torch.float32),     # two K chunks, the second of one step
     (4096, 70, 32, 49, torch.bfloat16),    # three K chunks
     (640, 5, 160, 300, torch.float32),     # down: a 128-row tile of 44 tokens, H in a short last column tile
