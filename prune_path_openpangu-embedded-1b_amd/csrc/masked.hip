@@ -26,21 +26,31 @@
 #define MG_THREADS 256
 #define MG_MAX_I 16384  // LDS holds one row's fp32 products; places in the expert-sorted order are 16-bit
 
-// 16-byte loads and stores. Results are stored non-temporally: they are read next by another
-// kernel, after 100s of MB, and stored normally they take the place of the rows this launch still
-// has to read (16384 x 6144 bf16: forward 79.5 -> 57.3 us on rows that the cache could
-// hold). The backward is its rows' last reader and loads them non-temporally too (forward and
-// backward together 191 -> 175.7 us, 5.75 TB/s; the forward's loads left normal: 184.8 with them
-// non-temporal, as its backward reads them again).
+// 16-byte loads and stores, non-temporal (NT) or not. A non-temporal result does not take the
+// place of rows that the launch still has to read, but the kernel that reads it next finds it in
+// memory, not in the cache.
+// Forward: NT where a result is larger than half of the 256 MB last-level cache (MG_NT_BYTES), so
+// that rows and results together do not fit. I = 6144, us, rows normal / NT: forward alone bf16
+// 1024 4.7 / 4.0, 16384 77 / 57; with an elementwise kernel before and a product with a [1536][I]
+// matrix after it bf16 512 30.6 / 34.0, 1024 41.9 / 46.4, 4096 106 / 111, 8192 202 / 204, 16384
+// 407 / 409 (followed by an elementwise kernel alone 183 / 178), fp32 6144 931 / 932 (142 / 140).
+// Backward: NT loads and stores at every size. It is its rows' last reader and stores as it reads;
+// between an elementwise kernel that writes d_out and one that reads d_inter, bf16 rows, normal
+// and NT: 512 24.2 / 20.0, 1024 31.2 / 32.5, 4096 80.6 / 81.7, 8192 168 / 153, 16384 332 / 313.
+#define MG_NT_BYTES ((int64_t)128 << 20)
 typedef uint32_t mg_u4 __attribute__((ext_vector_type(4)));
 template <bool NT>
 __device__ __forceinline__ uint4 mg_ld(const void* p) {
   const mg_u4 v = NT ? __builtin_nontemporal_load((const mg_u4*)p) : *(const mg_u4*)p;
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+template <bool NT>
 __device__ __forceinline__ void mg_st(void* p, uint4 u) {
   const mg_u4 v = {u.x, u.y, u.z, u.w};
-  __builtin_nontemporal_store(v, (mg_u4*)p);
+  if (NT)
+    __builtin_nontemporal_store(v, (mg_u4*)p);
+  else
+    *(mg_u4*)p = v;
 }
 
 template <typename T>
@@ -51,9 +61,10 @@ struct MgVec<float> {
     const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
   }
+  template <bool NT>
   static __device__ __forceinline__ void store(float* p, const float (&v)[8]) {
-    mg_st(p, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
-    mg_st(p + 4, make_uint4(__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7])));
+    mg_st<NT>(p, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
+    mg_st<NT>(p + 4, make_uint4(__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7])));
   }
   static __device__ __forceinline__ float gate(float g) { return g; }
 };
@@ -68,13 +79,14 @@ struct MgVec<bf16_t> {
       v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
     }
   }
+  template <bool NT>
   static __device__ __forceinline__ void store(bf16_t* p, const float (&v)[8]) {
     uint4 u;
     u.x = (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
     u.y = (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
     u.z = (uint32_t)f32_to_bf16(v[4]) | ((uint32_t)f32_to_bf16(v[5]) << 16);
     u.w = (uint32_t)f32_to_bf16(v[6]) | ((uint32_t)f32_to_bf16(v[7]) << 16);
-    mg_st(p, u);
+    mg_st<NT>(p, u);
   }
   static __device__ __forceinline__ float gate(float g) { return bf16_to_f32(f32_to_bf16(g)); }
 };
@@ -103,9 +115,9 @@ struct MgRow {
   }
 };
 
-// The forward takes one row per workgroup (no barrier between rows; the ids come
-// through L2 as int32 -- measured a little faster than the persistent form with the ids
-// in LDS, 80 against 85 us for 16384 x 6144 bf16).
+// The forward takes one row per workgroup (no barrier between rows; the ids come through L2 as
+// int32): 57 us for 16384 x 6144 bf16, 7.0 TB/s. The persistent form with the ids in LDS was a
+// little slower (85 against 80 us, both with normal stores).
 __device__ __forceinline__ void mg_eids(const int32_t* eid, int d, int E, int (&e)[8]) {
   const int4 a = *(const int4*)(eid + d), b = *(const int4*)(eid + d + 4);
   const int v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -113,7 +125,7 @@ __device__ __forceinline__ void mg_eids(const int32_t* eid, int d, int E, int (&
   for (int i = 0; i < 8; ++i) e[i] = (int)min((unsigned)v[i], (unsigned)(E - 1));  // clamped
 }
 
-template <typename T>
+template <typename T, bool NT>
 __global__ __launch_bounds__(MG_THREADS) void masked_gate_fwd_kernel(const T* __restrict__ inter,
                                                                      const float* __restrict__ gates,
                                                                      const int32_t* __restrict__ eid, int I, int E,
@@ -132,7 +144,7 @@ __global__ __launch_bounds__(MG_THREADS) void masked_gate_fwd_kernel(const T* __
     mg_eids(eid, d, E, e);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = __fmul_rn(v[i], g_s[e[i]]);
-    MgVec<T>::store(out + n * I + d, v);
+    MgVec<T>::template store<NT>(out + n * I + d, v);
   }
 }
 
@@ -222,7 +234,7 @@ __global__ __launch_bounds__(MG_THREADS, mg_bwd_wpc<T>(NI)) void masked_gate_bwd
           gi[i] = __fmul_rn(a[i], g[(ids[it][i >> 2] >> (8 * (i & 3))) & 0xff]);
           prod_s[(inv[it][i >> 1] >> (16 * (i & 1))) & 0xffff] = __fmul_rn(a[i], b[i]);
         }
-        if (d_inter) MgVec<T>::store(d_inter + n * I + d, gi);
+        if (d_inter) MgVec<T>::template store<true>(d_inter + n * I + d, gi);
       }
     }
     if (n + gridDim.x < n_rows) load(n + gridDim.x);
@@ -295,12 +307,18 @@ extern "C" int pp_masked_gate_fwd(const void* inter, int dtype, const float* gat
   PP_REQUIRE(inter && gates && expert_ids && out, PP_ERR_INVALID, "pp_masked_gate_fwd: null pointer");
   PP_REQUIRE(((uintptr_t)expert_ids & 15) == 0, PP_ERR_INVALID, "pp_masked_gate_fwd: expert_ids not 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == PP_DTYPE_F32)
-    masked_gate_fwd_kernel<float><<<(unsigned)n_rows, MG_THREADS, 0, st>>>((const float*)inter, gates, expert_ids, I,
-                                                                           E, (float*)out);
-  else
-    masked_gate_fwd_kernel<bf16_t><<<(unsigned)n_rows, MG_THREADS, 0, st>>>((const bf16_t*)inter, gates, expert_ids,
-                                                                            I, E, (bf16_t*)out);
+  const bool nt = n_rows * I * (dtype == PP_DTYPE_F32 ? 4 : 2) > MG_NT_BYTES;
+#define MG_FWD(T, NT)                                                                                                \
+  masked_gate_fwd_kernel<T, NT>                                                                                      \
+      <<<(unsigned)n_rows, MG_THREADS, 0, st>>>((const T*)inter, gates, expert_ids, I, E, (T*)out)
+  if (dtype == PP_DTYPE_F32) {
+    if (nt) MG_FWD(float, true);
+    else MG_FWD(float, false);
+  } else {
+    if (nt) MG_FWD(bf16_t, true);
+    else MG_FWD(bf16_t, false);
+  }
+#undef MG_FWD
   return pp_check_launch("pp_masked_gate_fwd");
 }
 

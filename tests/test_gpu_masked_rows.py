@@ -37,3 +37,18 @@ def test_masked_gate_bwd_rows(pkg, N, I, E, dtype):
     assert bool((err <= (prod.abs() @ onehot) * m.clamp(min=1) * 2.0 ** -24).all())
     none, again = pkg.ops.masked_gate_bwd(d, x, gates, *layout, need_d_inter=False)
     assert none is None and torch.equal(again, d_gates)
+
+
+@pytest.mark.parametrize("dtype,N", [(torch.float32, 2048), (torch.float32, 2049), (torch.bfloat16, 4096),
+                                     (torch.bfloat16, 4097)])
+def test_masked_gate_fwd_rows(pkg, dtype, N):
+    """The forward up to 128 MiB of rows and above, where its results are stored non-temporally:
+    bit for bit against the products."""
+    I, E = 16384, 37
+    g = torch.Generator(device=dev()).manual_seed(N)
+    x = torch.randn(N, I, device=dev(), generator=g).to(dtype)
+    gates = torch.rand(N, E, device=dev(), generator=g)
+    ids = torch.randint(E, (I,), device=dev(), generator=g)
+    want = (x.float() * gates.to(dtype).float()[:, ids]).to(dtype)
+    eid = pkg.ops.masked_gate_layout(ids, E)[0]
+    assert torch.equal(pkg.ops.masked_gate_fwd(x, gates, eid), want)
