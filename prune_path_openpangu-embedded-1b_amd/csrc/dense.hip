@@ -1141,6 +1141,9 @@ static int dense_pass(const void* x, int x_dtype, int64_t n, int H, const float*
 // pp_dense_split_words words, zero at launch; part: pp_dense_split_bytes.
 size_t pp_dense_split_bytes() { return (size_t)DG_MAX_GRID * DG_SLOT_BYTES; }
 int pp_dense_split_words() { return DG_SYNC_WORDS / 2; }
+int64_t pp_dense_down_tiles(int64_t n, int H) {  // of pp_dense_down
+  return (n + DG_DN_BM - 1) / DG_DN_BM * ((H + DG_DN_BN - 1) / DG_DN_BN);
+}
 int pp_dense_down(const bf16_t* act, int64_t n, int H, int E, int G, const bf16_t* down_t, bf16_t* out,
                   uint32_t* sync, float* part, const int32_t* meta, int min_pairs, const uint8_t* mask,
                   const float* y, const int32_t* token_pairs, const int32_t* count, hipStream_t st) {

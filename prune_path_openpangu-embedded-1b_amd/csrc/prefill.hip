@@ -934,6 +934,7 @@ int pp_bucket_impl(const uint8_t* mask, const float* gates, int64_t N, int E, in
 
 size_t pp_dense_split_bytes();
 int pp_dense_split_words();
+int64_t pp_dense_down_tiles(int64_t n, int H);
 int pp_dense_down(const bf16_t* act, int64_t n, int H, int E, int G, const bf16_t* down_t, bf16_t* out,
                   uint32_t* sync, float* part, const int32_t* meta, int min_pairs, const uint8_t* mask,
                   const float* y, const int32_t* token_pairs, const int32_t* count, hipStream_t st);
@@ -962,14 +963,30 @@ struct PrefillWs {
 // The line: at 4096 tokens the grouped side is faster at 38 % of the pairs (198 against 212 us),
 // the product at 52 % (237 against 250); at 2048 and 3072, where the product is cut into K ranges
 // and joined, at 52 % (140 / 153, 187 / 202) and 80 % (188 / 170, 267 / 243).
+//
+// Few of the product's 256 x 192 tiles (all cut in K, some workgroups idle) leave it no faster
+// where y is small too: from 64 tiles at H >= 1536 or G <= 128, 80 at H >= 768, 112 below. Layer
+// at 75 % and 90 % of the pairs, grouped / product, G = 384: H = 1024 66 tiles (2600 tokens) 138 /
+// 153 and 166 / 162, 84 177 / 171 and 217 / 183; H = 896 70 160 / 164 and 188 / 174, 80 180 / 171
+// and 221 / 190; H = 640 80 168 / 173 and 202 / 188, 96 199 / 210 and 246 / 226, 112 232 / 223 and
+// 290 / 248; H = 512 48 118 / 130 and 141 / 141. G = 64: H = 640 64 71 / 71 and 80 / 72, H = 896
+// 70 80 / 76 and 91 / 77, H = 512 48 62 / 66 and 70 / 67, 72 84 / 82 and 98 / 84.
+// Below PF_ALL_TAU a call of as many passes as before is offered it only where the line is the
+// lower one (passes of 4096 tokens): elsewhere the grouped side is likely, and the choice its cost
+// (H = 2560, 6500 tokens, tau 0.7 280 / 281 at G = 128, 458 / 472 at G = 384). Longer passes at other
+// widths, tau 0.5 / 0.7 / 0.8: H = 3072, G = 384, 8191 tokens 483 / 794 / 1017 -> 444 / 727 / 728,
+// H = 4096 639 / 1056 / 1327 -> 571 / 1009 / 1351, H = 2048, G = 128, 6500 tokens 161 / 228 / 299 ->
+// 132 / 244 / 189 (the grouped side of a pass of 6500 tokens costs more there than two of its halves).
 #define PF_ALL_MIN 2048
 #define PF_ALL_TAU 0.9f
+#define PF_ALL_LONG 4096  // tokens of a pass from which the lower line holds
+static int all_min_tiles(int H, int G) { return H >= 1536 || G <= 128 ? 64 : H >= 768 ? 80 : 112; }
 // Wider experts have more products per y row: a pair's grouped time is taken as
 // proportional to 2.67 G + 1780 (its products at the grouped GEMM's rate, its row at the memory's), its
 // share of the whole product to 2 G, and the line above, measured at G = 384, moves with their
 // ratio; at 100 % (G >= 2944, below 4096 tokens G >= 896) the form is not offered.
 static int all_pct(int64_t n, int G) {
-  const double base = n < 4096 ? 65.0 : 45.0, w = G > 384 ? G : 384;
+  const double base = n < PF_ALL_LONG ? 65.0 : 45.0, w = G > 384 ? G : 384;
   return (int)std::min(100.0, base * (w / (2.67 * w + 1780.0)) / (384.0 / (2.67 * 384.0 + 1780.0)));
 }
 static int all_min_pairs(int64_t n, int E, int pct) { return (int)(n * E * pct / 100); }
@@ -1041,9 +1058,12 @@ static PrefillPlan prefill_plan(int64_t N, int H, int E, int G, float tau) {
     return n > 0 && !prefill_short_tiles(n, H, G) && pp_bucket_counts_fit(n, E, pp_route_count_block(n, H, E)) &&
            prefill_layout(n, H, E, G, pct).total <= have;
   };
-  for (int64_t k = 1; k <= (N + ng - 1) / ng && N / k >= PF_ALL_MIN; ++k) {  // no more passes than grouped
+  const int64_t kg = (N + ng - 1) / ng;
+  for (int64_t k = 1; k <= kg && N / k >= PF_ALL_MIN; ++k) {  // no more passes than grouped
     const int64_t n = ((N + k - 1) / k + 3) / 4 * 4;  // (mask rows of every pass 4-byte aligned)
     const int64_t first = min(n, N);
+    if (pp_dense_down_tiles(first, H) < all_min_tiles(H, G)) break;  // (fewer with every k)
+    if (k == kg && !(tau >= PF_ALL_TAU) && first < PF_ALL_LONG) break;
     const int pct = all_pct(first, G);
     if (pct < 100 && fits(first, pct) && fits(N - (k - 1) * n, pct)) return {n, pct};
   }

@@ -43,7 +43,7 @@ def offered(pkg, N, H, tau, mask, taken):
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("H,N", [
-    (512, 4100),   # 17 x 3 tiles, all of them cut in K
+    (512, 5399),   # 22 x 3 tiles, all of them cut in K
     (1664, 8192),  # 32 x 9 tiles: one round of whole tiles, the rest cut in K
 ])
 def test_prefill_all_experts_nonfinite_weights(pkg, H, N, bad):

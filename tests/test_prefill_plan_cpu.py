@@ -51,3 +51,18 @@ def test_no_plan_for_other_shapes():
     for N, H, E, G in [(0, 1536, 16, 384), (-1, 1536, 16, 384), (16, 100, 16, 384), (16, 1536, 192, 32),
                        (0x7fffffff // 256 + 1, 1536, 16, 384)]:
         assert lib.pp_prefill_pass(N, H, E, G, 0.7, 0, None, None, None) == 0
+
+
+@pytest.mark.parametrize("H,G,N,tau,passes,offered", [
+    (1536, 384, 2047, 0.95, 1, False), (1536, 384, 2048, 0.95, 1, True), (1536, 384, 2048, 0.89, 1, False),
+    (1536, 384, 8191, 0.5, 1, True),                                     # one pass less
+    (1024, 384, 2600, 0.95, 1, False), (1024, 384, 3500, 0.95, 1, True),   # 66 and 84 tiles
+    (640, 384, 6000, 0.95, 1, False), (640, 384, 7000, 0.95, 1, True),   # 96 and 112 tiles
+    (1024, 64, 2600, 0.95, 1, True),
+    (2560, 384, 6500, 0.7, 2, False), (2560, 384, 6500, 0.95, 2, True),  # as many passes as grouped
+    (2560, 384, 8191, 0.7, 2, True),                                     # one less; 4096 tokens a pass
+])
+def test_where_the_product_is_offered(H, G, N, tau, passes, offered):
+    p = prefill_passes(import_pkg()._lib.lib(), N, H, 16, G, tau)
+    assert len(p) == passes
+    assert all((m >= 0) == offered for _, m, _ in p)
