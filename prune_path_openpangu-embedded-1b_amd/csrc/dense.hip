@@ -1021,18 +1021,23 @@ static int dense_blocks(int64_t tiles, int nkb) {
 }
 
 // down: 128-row tiles where 256-row tiles would all be cut in K, unless the parts they can be cut
-// into leave them more than twice the K blocks. A block of theirs takes about half the time (three
-// stages in flight instead of two), their partial sums are half the bytes to join, and up to 128
-// tokens of padding go. E = 192, G = 32, H = 1536, layer, us, 256- and 128-row tiles: 84.2 / 67.9
-// at 257 tokens, 87.2 / 76.8 at 509, 123.7 / 116.1 at 1024, 286.5 / 275.3 at 4096; more than
-// twice the blocks: 153.2 / 154.7 at 1536, and 495 / 534 at E = 200, G = 160, H = 4096, 500 tokens.
+// into leave them more than 1.75 times the K blocks and 12 (what the smaller join saves), at most
+// twice. A block of theirs takes about half the time (three stages in flight instead of two), their
+// partial sums are half the bytes to join, and up to 128 tokens of padding go. Layer, us, 256- and
+// 128-row tiles, E = 192, G = 32: H = 1536 85.6 / 65.1 at 257 tokens, 88.6 / 74.0 at 509, 120.5 /
+// 115.1 at 1024, 162.8 / 160.7 at 2048, 272 / 266 at 4096 (the last three twice the blocks), H =
+// 4096 241 / 230 at 1024 (48 and 96 blocks); more than twice: H = 1536 153.2 / 154.7 at 1536 tokens.
+// Long K, E = 200, G = 160, twice the blocks: H = 2048 868 / 931 at 1800 tokens (250 and 500), H =
+// 3072 603 / 628 at 900 (125 and 250), H = 4096 867 / 933 at 1024; fewer: H = 4096 643 / 618 at 513
+// (167 and 250).
 // Whole 256-row tiles stay: their operands cross L2 half as often (8191 tokens of the E = 16
 // prefill's product 466 / 505).
 static bool down_short_tiles(int64_t n, int H, int Ipad) {
   const int64_t ct = (H + DG_DN_BN - 1) / DG_DN_BN;
   const int64_t t256 = (n + DG_DN_BM - 1) / DG_DN_BM * ct, t128 = (n + DG_DS_BM - 1) / DG_DS_BM * ct;
   const int nkb = Ipad / DG_DN_BK;
-  return 2 * t256 <= dense_grid() && dense_blocks(t128, nkb) <= 2 * dense_blocks(t256, nkb);
+  const int b256 = dense_blocks(t256, nkb), b128 = dense_blocks(t128, nkb);
+  return 2 * t256 <= dense_grid() && 4 * b128 <= std::min(8 * b256, 7 * b256 + 48);
 }
 
 // One pass over n tokens (at most dense_pass_tokens). logits_out / mask_out (may be null)
