@@ -974,13 +974,18 @@ static FewWs few_layout(int64_t n, int H, int I) {
   return L;
 }
 
-// E = 192, G = 32, H = 1536, layer, us, GEMM tiles and this form: 83 / 27 at 2 tokens, 82 / 28.7 at
-// 16, 84 / 37.7 at 64, 67.6 / 49.5 at 128 (128-row down tiles), 69.0 / 61.4 at 192, 70.3 / 67.1 at
-// 224, 70.7 / 72.9 at 256; at H = 512 53.4 / 45.7 at 200. H > 1536: the
-// weights no longer stay in registers over more than 64 tokens (H = 4096: 107 -> 84 at 64, 123 ->
-// 124 at 128). Buffers in the GEMMs' split workspace, which such a pass does not use.
+// Layer, us, GEMM tiles and this form, E = 192, G = 32: H = 1536 83 / 27 at 2 tokens, 82 / 28.0 at
+// 16, 84 / 36.6 at 64, 67.6 / 48.3 at 128 (128-row down tiles), 69.0 / 61.4 at 192, 70.3 / 67.1 at
+// 224, 70.7 / 72.9 at 256; H = 512 65.0 / 48.4 at 224. H > 1536: the weights no longer stay in
+// registers over more than 64 tokens (H = 4096: 107 -> 84 at 64, 123 -> 124 at 128). H < 512: little
+// weight to stream, and the form's tokens cost more than the GEMM's: H = 128 46.7 / 44.5 at 192,
+// 47.0 / 50.4 at 224, and with the selection in a launch of its own (E <= 64) E = 64 67.3 / 68.2 at
+// 160, 67.3 / 72.2 at 192 (H = 384 73.0 / 70.3, 72.7 / 75.3).
+static int dense_few_max(int H, int E) { return H > 1536 ? 64 : H >= 512 ? DF_MAX : E > 64 ? 192 : 160; }
+
+// Buffers in the GEMMs' split workspace, which such a pass does not use.
 static bool dense_few_form(int64_t n, int H, int E, int G) {
-  return E != 16 && n <= (H <= 1536 ? DF_MAX : 64) &&
+  return E != 16 && n <= dense_few_max(H, E) &&
          few_layout(n, H, E * G).total * 4 <= (int64_t)DG_MAX_GRID * (int64_t)DG_SLOT_BYTES;
 }
 

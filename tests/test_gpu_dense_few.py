@@ -29,6 +29,8 @@ pytestmark = pytest.mark.gpu
     (768, 24, 32, 16, torch.float32),      # three
     (1024, 5, 160, 100, torch.bfloat16),   # four
     (1280, 100, 32, 17, torch.float32),    # five
+    (128, 70, 32, 192, torch.float32),     # the largest batch below H = 512
+    (384, 64, 32, 161, torch.bfloat16),    # above it with the selection apart: GEMM tiles
     (640, 200, 32, 129, torch.bfloat16),   # two groups of token blocks on weights loaded once
     (1664, 20, 96, 64, torch.float32),     # two K chunks, the second of one step
     (4096, 70, 32, 49, torch.bfloat16),    # three K chunks
