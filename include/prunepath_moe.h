@@ -250,15 +250,18 @@ int pp_moe_decode_batch(const void* x, int x_dtype, int64_t n_tokens, int H, con
  *     one pass at E = 16, H = 1536). At E = 16, calls longer than that (and from 2048 tokens
  *     on with tau >= 0.9) may instead take one down GEMM over every expert, the acts of the
  *     experts a token does not select being 0: chosen on the device, per pass, from the
- *     number of selected pairs; passes of up to 8192 tokens on the same workspace.
+ *     number of selected pairs; passes of up to 8192 tokens on the same workspace, where their
+ *     buffers fit it and the call is large enough (pp_prefill_pass tells both).
  *   G % 64 != 0 (e.g. the checkpoint's E = 192 experts of G = 32 neurons, narrower than an
  *     MFMA column tile): router logits (fp32 MFMA, one fixed summation order per
  *     (token, expert): a token routes the same way in any batch) -> selection -> dense
  *     gate/up GEMM over every (token, neuron) with act = bf16(silu(g) * u * gate), 0 for the
  *     experts a token does not select -> dense down GEMM over all neurons, fp32
- *     accumulation, one rounding to bf16. Up to 224 tokens (64 above H = 1536): the same
- *     arithmetic in three launches that stream the weights. Passes of up to ~256 MiB of
- *     per-token buffers (about 15000 tokens at H = 1536, E = 192, G = 32).
+ *     accumulation, one rounding to bf16. Small batches (E != 16; up to 224 tokens at
+ *     512 <= H <= 1536, 64 above, below 192, or 160 with E <= 64; and buffers that fit the
+ *     GEMMs' split workspace) take the same arithmetic, summed in another order, in three
+ *     launches that stream the weights (four with E <= 64: the selection apart). Passes of up
+ *     to ~256 MiB of per-token buffers (about 15000 tokens at H = 1536, E = 192, G = 32).
  * Either way every token's routing is the same as in one pass over all N (its sums may be
  * taken in another order), and the output is the same bits on every call with the same N.
  * workspace: pp_prefill_workspace_bytes(N, H, E, G) bytes of device scratch.

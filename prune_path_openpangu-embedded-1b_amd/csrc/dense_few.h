@@ -12,8 +12,8 @@
 //                             workgroups of the same launch, one token each
 //   dense_few_down_kernel     act = bf16(h * gate), 0 where the expert is not selected (as
 //                             dense_gemm_kernel<0>'s epilogue), out = bf16(act . Wd)
-// What bounds it: at 16 tokens the three launches take about 8, 11 and 9 us (82 us before, on
-// the GEMM tiles), of which a stream of the weights at the rate of a large copy would be 9 us:
+// What bounds it: at 16 tokens the three launches take about 9.5 us each, 28 in all (82 us before,
+// on the GEMM tiles), of which a stream of the weights at the rate of a large copy would be 9 us:
 // the logits are one latency chain (router rows from memory, 96 dependent MFMAs), the other
 // two a launch, a cold stream and the sums of the waves. Beyond, each 16 tokens cost ~2.9 us:
 // x and h pass once per workgroup through L2, and the sums once through LDS. Two token tiles per
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256, 1) void route_logits_few_kernel(const XT* __re
 }
 
 // ------------------------------------------------------------------ gate/up
-#define DF_MAX 224  // tokens at most (dense_few_form)
+#define DF_MAX 224  // tokens at most (dense_few_max)
 
 struct FewArgs {
   const bf16_t* xfrag;    // x as bf16: [H / 32][token block][lane][8]

@@ -575,7 +575,7 @@ __device__ __forceinline__ void gemm_v3_body(
 // items, and three stages where the wide tile has two. With a workgroup alone on its CU a K block
 // is a DMA latency, not bandwidth or MFMA work: at E = 16, G = 384, H = 1536 the gate/up launch
 // takes 27 -> 17.5 us at 128 tokens (96 wide items; two stages 24, four or six 17), 28 -> 25.4 at 333
-// (144: some CUs then hold two narrow items), the layer 56.1 -> 45.4 and 54.0 -> 50.5; from 192
+// (144: some CUs then hold two narrow items), the layer 50.2 -> 42.4 and 56.8 -> 52.8; from 192
 // wide items (500 tokens) on both take the same, past one per CU the narrow tile's second
 // reading of A costs (800 tokens 72.7 -> 75.4).
 // NARROW and ALL (the down projection over every expert may follow) are template parameters, so
@@ -984,7 +984,10 @@ static int all_min_tiles(int H, int G) { return H >= 1536 || G <= 128 ? 64 : H >
 // Wider experts have more products per y row: a pair's grouped time is taken as
 // proportional to 2.67 G + 1780 (its products at the grouped GEMM's rate, its row at the memory's), its
 // share of the whole product to 2 G, and the line above, measured at G = 384, moves with their
-// ratio; at 100 % (G >= 2944, below 4096 tokens G >= 896) the form is not offered.
+// ratio; at 100 % (G >= 2944, below 4096 tokens G >= 896) the form is not offered. At 75 % and 90 % of
+// the pairs, grouped / this form, H = 1536, 4096 tokens: G = 64 139 / 96 and 187 / 98, G = 768 481 / 443
+// and 599 / 503, G = 1024 (line at 74 %) 603 / 609 and 757 / 662; H = 2560, G = 512, 3001 tokens (line
+// at 77 %, so the grouped side at 75 %) 455 / 459 and 565 / 456, 6000 in two passes 891 / 920 and 1108 / 901.
 static int all_pct(int64_t n, int G) {
   const double base = n < PF_ALL_LONG ? 65.0 : 45.0, w = G > 384 ? G : 384;
   return (int)std::min(100.0, base * (w / (2.67 * w + 1780.0)) / (384.0 / (2.67 * 384.0 + 1780.0)));
